@@ -90,7 +90,7 @@ ScratchW& batch_scratch(Batch& b, size_t i, int W) {
         const DeviceOp& op = *b.ops[i];
         const size_t sb = static_cast<size_t>(staging(op, W).bytes);
         HIPCHECK(hipMalloc(&s.S, sb));
-        HIPCHECK(hipMemset(s.S, 0, sb));
+        zero_staging_tail(s.S, staging(op, W), nullptr);
         HIPCHECK(hipMalloc(&s.P, std::max<int64_t>(op.npartial, 1) * W * p_elem(op.storage)));
         HIPCHECK(hipMalloc(&s.LP, std::max<int64_t>(op.nlpartial, 1) * W * p_elem(op.storage)));
         HIPCHECK(hipMalloc(&s.Yp, std::max<int64_t>(op.m, 1) * W * p_elem(op.storage)));
@@ -148,6 +148,7 @@ void build_lists(Batch& b) {
         d.nrhs = b.nrhs;
         d.rhs0 = 0;
     }
+    HIPCHECK(hipStreamSynchronize(nullptr));  // the scratch is cleared before any stream reads it
     std::stable_sort(A.begin(), A.end(), [](const FarItem& x, const FarItem& y) {
         return int64_t(x.ktiles) * x.nrg > int64_t(y.ktiles) * y.nrg;
     });

@@ -664,7 +664,6 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
         const size_t yb = std::max<int64_t>(op.m, 1) * W * p_elem(op.storage);
         try {
             HIPCHECK(hipMalloc(&n.S, sb));
-            HIPCHECK(hipMemset(n.S, 0, sb));  // zero row and padding rows
             HIPCHECK(hipMalloc(&n.P, pb));
             HIPCHECK(hipMalloc(&n.LP, lb));
             HIPCHECK(hipMalloc(&n.Yp, yb));
@@ -673,6 +672,10 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
                 if (p) (void)hipFree(p);
             throw;
         }
+        // On the product's own stream: a clear on the null stream is not ordered
+        // before the work of a stream created without that dependence, and would
+        // overwrite rows that the first product has already written.
+        zero_staging_tail(n.S, staging(op, W), stream);
         s = n;
         it->second.bytes += sb + pb + lb + yb;
         if (std::getenv("HMX_VERBOSE"))
@@ -817,13 +820,6 @@ NoAllocPlan noalloc_plan(const DeviceOp& op, int W) {
     return pl;
 }
 
-// Zero n16 16-byte words (the zero row and padding rows of S: every call
-// clears them, since the previous call may have left other data there).
-__global__ __launch_bounds__(256) void k_zero16(uint4* __restrict__ p, int64_t n16) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n16) p[i] = make_uint4(0u, 0u, 0u, 0u);
-}
-
 template <typename TS, int W, typename TIO>
 void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs,
                  hipStream_t st, unsigned char* base, const NoAllocPlan& pl) {
@@ -847,13 +843,7 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
     one.s0 = op.s0;
     one.s_rows = static_cast<uint32_t>(lay.rows);
     one.nrhs = nrhs;
-    // rows n + R .. end of S (the zero row and the padding rows) must read 0;
-    // a row is W * s_elem bytes, a multiple of 16 for W >= 4 (W = 1: cleared
-    // from the 16-byte word that holds row n + R)
-    const size_t z0 = static_cast<size_t>(lay.zero_begin);
-    const int64_t n16 = (lay.zero_end - lay.zero_begin) / 16;
-    hipLaunchKernelGGL(k_zero16, dim3(static_cast<unsigned>((n16 + 255) / 256)), dim3(256), 0, st,
-                       reinterpret_cast<uint4*>(base + pl.s + z0), n16);
+    zero_staging_tail(base + pl.s, lay, st);
     StageArrays A;
     A.itemsA = op.itemsA;
     A.nA = op.nA;

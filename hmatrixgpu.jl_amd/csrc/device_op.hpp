@@ -59,6 +59,16 @@ struct DeviceOp {
 inline StagingLayout staging(const DeviceOp& op, int W) {
     return staging_layout(op.s0 + op.n, op.R, op.storage, W);
 }
+// Clear rows n + R .. end of S on `st`: the zero row and the padding rows must
+// read 0, every other row is written before it is read.  A row is W * s_elem
+// bytes, a multiple of 16 for W >= 4 (W = 1: cleared from the 16-byte word that
+// holds row n + R, before X and T are written).
+inline void zero_staging_tail(void* S, const StagingLayout& lay, hipStream_t st) {
+    const int64_t n16 = (lay.zero_end - lay.zero_begin) / 16;
+    hipLaunchKernelGGL(k_zero16, dim3(static_cast<unsigned>((n16 + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<uint4*>(static_cast<char*>(S) + lay.zero_begin), n16);
+    HIPCHECK(hipGetLastError());
+}
 // element size of the partial sums
 inline size_t p_elem(int storage) { return storage == HMX_F64 ? 8 : 4; }
 

@@ -802,6 +802,12 @@ __global__ __launch_bounds__(256) void k_gather(const InstDesc one, const InstDe
     reinterpret_cast<SRowOut<s_t, W>*>(I.S)[I.s0 + p] = row;
 }
 
+// Zero n16 16-byte words.
+static __global__ __launch_bounds__(256) void k_zero16(uint4* __restrict__ p, int64_t n16) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n16) p[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // ---- build-time panel generation ------------------------------------------------
 // Column descriptors of the leaf panels: kind 0 = built-in kernel entry
 // (base = 0-based original source index), 1 = U payload, 2 = dense payload (callback
