@@ -28,8 +28,8 @@
 //     a single RHS is a VALU GEMV over the same tiles.
 //
 // Stages per call (one launch each, stream ordered): gather X -> S, far-field
-// panels (V*X), partial reduce, leaf panels (near field + U*T) -> permuted
-// rows or piece partials, piece sum, unpermute -> Y.
+// panels (V*X), partial reduce, leaf panels (near field + U*T) -> leaf-result
+// rows, sum of each row's pieces -> Y.
 #include "device_op.hpp"
 
 #include <algorithm>
@@ -68,54 +68,79 @@ int64_t leaf_item_work(const PairItem& it) {
     return a * 64 + 4096;
 }
 
-// Cut leaf items whose panels exceed max(total / kLeafPieces, kMinPiece) bytes
-// into pieces along k (each of the shared and private k-tile ranges split in
-// proportion), so that the launch has several items per resident workgroup
-// and no single item outlasts the rest.  Pieces write partial rows; the
-// returned groups sum them in piece order.  Returns the partial rows used.
-constexpr int64_t kLeafPieces = 12288, kMinPiece = int64_t(1) << 20;
+// Size of the k-range pieces that leaf items are cut into, from the leaf bytes of
+// the operator: total / kLeafPieces, at least 1 MiB, so that no item outlasts the
+// launch (swept at N = 262,144).  An operator of at most kSmallLeaf bytes has fewer
+// whole items than the 1,024 workgroups that are resident; it takes total /
+// kSmallPieces, between 128 and 256 KiB.  Measured on the leaf kernel: N = 4,096
+// FP64 with one right-hand side 53 -> 29 us, FP32 with 16 43 -> 18 us; 64 KiB
+// pieces are slower again (start-up of each piece, about 5 us of one workgroup).
+// The line lies where a batch of such operators, which fills the GPU without
+// cutting its members (and must cut them as their own products do, for the same
+// bits), starts to pay for that start-up: 16 members of 2,048 .. 16,384 points take
+// 498 us with 1 MiB pieces, 500 us with this rule, 509 us with twice these limits.
+constexpr int64_t kLeafPieces = 12288, kSmallPieces = 512;
+constexpr int64_t kMiB = int64_t(1) << 20;
+constexpr int64_t kSmallLeaf = 160 * kMiB;
 constexpr int kMaxPieces = 64;
+// Target rows up to which an operator without cut items writes Y from the leaf
+// kernel: scattered stores, but one launch less (N = 1,000, one right-hand side:
+// 17.3 -> 14.5 us per product).
+constexpr int64_t kDirectRows = 8192;
 
-int64_t split_leaf_items(std::vector<PairItem>& items, int TK, int64_t pieces,
-                         std::vector<LeafGroup>& groups) {
-    int64_t total = 0;
-    for (const PairItem& it : items) total += leaf_item_work(it);
-    // HMX_LEAF_MIN_PIECE lowers the minimum piece (bytes), e.g. to split the
+int64_t leaf_piece_bytes(int64_t total, int64_t pieces) {
+    // HMX_LEAF_MIN_PIECE sets the smallest piece (bytes), e.g. to split the
     // items of small operators in tests
     const char* min_env = std::getenv("HMX_LEAF_MIN_PIECE");
-    const int64_t min_piece = min_env ? std::max<int64_t>(4096, std::atoll(min_env)) : kMinPiece;
-    const int64_t piece = std::max(total / pieces, min_piece);
+    const int64_t min_piece =
+        min_env ? std::max<int64_t>(4096, std::atoll(min_env))
+        : total > kSmallLeaf
+            ? kMiB
+            : std::min(kMiB / 4, std::max(kMiB / 8, total / kSmallPieces));
+    return std::max(total / pieces, min_piece);
+}
+
+// Cut the leaf items into pieces of about `piece` bytes along k, so that the
+// launch has several items per resident workgroup and no single item outlasts the rest.
+// Every piece gets its own leaf-result rows; `src` (per permuted target row)
+// says which rows to sum.  Returns the leaf-result rows used.
+int64_t split_leaf_items(std::vector<PairItem>& items, int TK, int64_t piece,
+                         std::vector<RowSrc>& src) {
     std::vector<PairItem> out;
     out.reserve(items.size());
     int64_t nrows = 0;
     for (const PairItem& it : items) {
-        const int64_t c = std::min<int64_t>(kMaxPieces, (leaf_item_work(it) + piece - 1) / piece);
-        if (c <= 1) {
-            out.push_back(it);
-            continue;
-        }
+        const int64_t c =
+            piece > 0 ? std::min<int64_t>(kMaxPieces, (leaf_item_work(it) + piece - 1) / piece) : 1;
         const int32_t rows = it.rows[0] + it.rows[1];
-        LeafGroup g{};
-        g.pbase = nrows;
-        g.out_off[0] = it.out_off[0];
-        g.out_off[1] = it.out_off[1];
-        g.rows[0] = it.rows[0];
-        g.rows[1] = it.rows[1];
-        g.nparts = static_cast<int32_t>(c);
-        g.inst = it.inst;
-        groups.push_back(g);
-        auto cut = [c](int32_t kt, int64_t p) { return static_cast<int32_t>(kt * p / c); };
+        for (int g = 0; g < 2; g++)
+            for (int32_t r = 0; r < it.rows[g]; r++)
+                src[it.out_off[g] + r] = RowSrc{static_cast<uint32_t>(nrows + g * it.rows[0] + r),
+                                                static_cast<int16_t>(c), static_cast<int16_t>(rows)};
+        // Piece boundaries along the work of the panels: the shared tiles (both
+        // row groups together), then the private ones in proportion.  Each piece
+        // is one contiguous k-range of each row group.
+        const int64_t wsh = int64_t(it.sh_kt) * rows;
+        const int64_t wpr = int64_t(it.pr_kt[0]) * it.rows[0] + int64_t(it.pr_kt[1]) * it.rows[1];
+        auto bound = [&](int64_t p, int32_t& sh, int32_t (&pr)[2]) {
+            const int64_t w = (wsh + wpr) * p / c;
+            sh = static_cast<int32_t>(std::min<int64_t>(it.sh_kt, w / rows));
+            for (int g = 0; g < 2; g++)
+                pr[g] = p == c     ? it.pr_kt[g]
+                        : w <= wsh ? 0
+                                   : static_cast<int32_t>(it.pr_kt[g] * (w - wsh) / wpr);
+        };
         for (int64_t p = 0; p < c; p++) {
             PairItem q = it;
-            const int32_t s0 = cut(it.sh_kt, p), s1 = cut(it.sh_kt, p + 1);
+            int32_t s0, s1, a0[2], a1[2];
+            bound(p, s0, a0);
+            bound(p + 1, s1, a1);
             q.sh_kt = s1 - s0;
             q.sh_col = it.sh_col + int64_t(s0) * TK;
             for (int gi = 0; gi < 2; gi++) {
-                const int32_t a0 = cut(it.pr_kt[gi], p), a1 = cut(it.pr_kt[gi], p + 1);
-                q.pr_kt[gi] = a1 - a0;
-                q.pr_col[gi] = it.pr_col[gi] + int64_t(a0) * TK;
-                q.sh_data[gi] = it.sh_data[gi] + int64_t(s0) * TK * it.rows[gi];
-                q.pr_data[gi] = it.pr_data[gi] + int64_t(a0) * TK * it.rows[gi];
+                q.pr_kt[gi] = a1[gi] - a0[gi];
+                q.pr_col[gi] = it.pr_col[gi] + int64_t(a0[gi]) * TK;
+                q.data[gi] = it.data[gi] + int64_t(s0 + a0[gi]) * TK * it.rows[gi];
             }
             q.part = nrows;
             nrows += rows;
@@ -182,18 +207,34 @@ void order_far_items(std::vector<FarItem>& items) {
     });
 }
 
+// Byte offsets of the three scratch arrays of one pass width inside the static
+// scratch of hmx_matvec_noalloc (each 256-byte aligned): S rows, far-field
+// partials, leaf-result rows.
+struct NoAllocPlan {
+    size_t s = 0, p = 0, lp = 0, total = 0;
+};
+NoAllocPlan noalloc_plan(const DeviceOp& op, int W) {
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t pe = p_elem(op.storage);
+    NoAllocPlan pl;
+    pl.s = 0;
+    pl.p = up(static_cast<size_t>(staging(op, W).bytes));
+    pl.lp = pl.p + up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe);
+    pl.total = pl.lp + up(static_cast<size_t>(std::max<int64_t>(op.nlrows, 1)) * W * pe);
+    return pl;
+}
+
 }  // namespace
 
 void device_destroy(DeviceOp* op) {
     if (!op) return;
     (void)hipSetDevice(op->device);
     for (void* p : {op->panel, (void*)op->itemsB, (void*)op->colidx, (void*)op->itemsA,
-                    (void*)op->groups, (void*)op->lgroups, (void*)op->tmap0, (void*)op->inv_tmap,
-                    (void*)op->inv_smap})
+                    (void*)op->groups, (void*)op->tmap0, (void*)op->rowsrc, (void*)op->inv_smap})
         if (p) (void)hipFree(p);
     for (auto& kv : op->scratch)
         for (auto& w : kv.second.w)
-            for (void* p : {w.S, w.P, w.LP, w.Yp})
+            for (void* p : {w.S, w.P, w.LP})
                 if (p) (void)hipFree(p);
     for (auto& e : op->ev)
         for (auto& pr : e) {
@@ -211,7 +252,7 @@ int64_t device_index_bytes(const DeviceOp* op) {
     return op->ncol * 4 + op->nA * static_cast<int64_t>(sizeof(FarItem)) +
            op->nB * static_cast<int64_t>(sizeof(PairItem)) +
            op->nG * static_cast<int64_t>(sizeof(ReduceGroup)) +
-           op->nLG * static_cast<int64_t>(sizeof(LeafGroup)) + (2 * op->m + op->n) * 4;
+           op->m * static_cast<int64_t>(4 + sizeof(RowSrc)) + op->n * 4;
 }
 
 // Build the device operator for one storage precision.
@@ -489,7 +530,7 @@ void device_build(HMatrix& h, int storage) {
             auto [c0, kt] = add_colidx(dense_of[A.leaf], lr_of[A.leaf]);
             it.pr_col[0] = c0;
             it.pr_kt[0] = kt;
-            it.pr_data[0] = add_panel(dense_of[A.leaf], lr_of[A.leaf], A);
+            it.data[0] = add_panel(dense_of[A.leaf], lr_of[A.leaf], A);
         } else {
             const Unit& B = units[gp.second];
             it.out_off[1] = B.r0;
@@ -499,18 +540,18 @@ void device_build(HMatrix& h, int storage) {
             auto [sc, skt] = add_colidx(sd.first, sl);
             it.sh_col = sc;
             it.sh_kt = skt;
-            it.sh_data[0] = add_panel(sd.first, sl, A);
-            it.sh_data[1] = add_panel(sd.second, sl, B);
             const Unit* UU[2] = {&A, &B};
-            std::vector<int32_t>* sdq[2] = {&sd.first, &sd.second};
+            const std::vector<int32_t> sdq[2] = {sd.first, sd.second};
             for (int q = 0; q < 2; q++) {
-                std::sort(sdq[q]->begin(), sdq[q]->end());
-                const auto pd = minus(dense_of[UU[q]->leaf], *sdq[q]);
+                it.data[q] = add_panel(sdq[q], sl, *UU[q]);
+                std::vector<int32_t> matched = sdq[q];
+                std::sort(matched.begin(), matched.end());
+                const auto pd = minus(dense_of[UU[q]->leaf], matched);
                 const auto pl = minus(lr_of[UU[q]->leaf], sl);
                 auto [pc, pkt] = add_colidx(pd, pl);
                 it.pr_col[q] = pc;
                 it.pr_kt[q] = pkt;
-                it.pr_data[q] = add_panel(pd, pl, *UU[q]);
+                add_panel(pd, pl, *UU[q]);
             }
         }
         itemsB.push_back(it);
@@ -520,12 +561,10 @@ void device_build(HMatrix& h, int storage) {
     op->npartial = npartial;
 
     // -- upload and generate ---------------------------------------------------------
-    std::vector<int32_t> tmap0(h.m), inv_t(h.m), inv(h.n);
+    std::vector<int32_t> tmap0(h.m), inv(h.n);
     for (int64_t i = 0; i < h.m; i++) tmap0[i] = static_cast<int32_t>(h.tmap[i] - 1);
-    for (int64_t i = 0; i < h.m; i++) inv_t[h.tmap[i] - 1] = static_cast<int32_t>(i);
     for (int64_t i = 0; i < h.n; i++) inv[h.smap[i] - 1] = static_cast<int32_t>(i);
     op->tmap0 = upload(tmap0);
-    op->inv_tmap = upload(inv_t);
     op->inv_smap = upload(inv);
     // The FP64 staging arrays are allocated before the panel and freed after
     // generation.  Measured on the MI355X, the product's speed depends on where
@@ -591,14 +630,45 @@ void device_build(HMatrix& h, int storage) {
         if (p) (void)hipFree(p);
 
     // HMX_LEAF_PIECES: target piece count of the split (0 keeps every leaf item whole)
-    std::vector<LeafGroup> lgroups;
     const char* pieces_env = std::getenv("HMX_LEAF_PIECES");
     const int64_t pieces = pieces_env ? std::atoll(pieces_env) : kLeafPieces;
-    if (pieces > 0) op->nlpartial = split_leaf_items(itemsB, TK, pieces, lgroups);
+    int64_t leaf_bytes = 0;
+    for (const PairItem& it : itemsB) leaf_bytes += leaf_item_work(it);
+    std::vector<RowSrc> src(h.m);
+    const size_t whole = itemsB.size();
+    const std::vector<PairItem> uncut = itemsB;
+    op->nlrows = split_leaf_items(itemsB, TK, pieces > 0 ? leaf_piece_bytes(leaf_bytes, pieces) : 0, src);
+    {
+        // the finer pieces of a smaller operator must not push a product past the
+        // static scratch of hmx_matvec_noalloc
+        std::vector<PairItem> coarse = uncut;
+        std::vector<RowSrc> csrc(h.m);
+        const int64_t fine_rows = op->nlrows;
+        const int64_t rows = split_leaf_items(
+            coarse, TK, pieces > 0 ? std::max(leaf_bytes / pieces, kMiB) : 0, csrc);
+        bool refused = false;
+        for (int W : {1, 4, 16}) {
+            op->nlrows = fine_rows;
+            const bool fine_fits = noalloc_plan(*op, W).total <= kNoAllocScratchBytes;
+            op->nlrows = rows;
+            refused = refused || (!fine_fits && noalloc_plan(*op, W).total <= kNoAllocScratchBytes);
+        }
+        if (refused) {
+            itemsB.swap(coarse);
+            src.swap(csrc);
+        } else {
+            op->nlrows = fine_rows;
+        }
+    }
+    op->direct = itemsB.size() == whole && h.m <= kDirectRows;
+    {
+        std::vector<RowSrc> by_row(h.m);  // permuted -> original target rows
+        for (int64_t i = 0; i < h.m; i++) by_row[tmap0[i]] = src[i];
+        op->rowsrc = upload(by_row);
+    }
     op->hItemsA = itemsF;  // tree order, for batched operators
     op->hItemsB = itemsB;
     op->hGroups = groups;
-    op->hLGroups = lgroups;
     order_far_items(itemsF);
     const char* order_env = std::getenv("HMX_ITEM_ORDER");
     order_leaf_items(itemsB, order_env ? order_env : "xcd");
@@ -608,8 +678,6 @@ void device_build(HMatrix& h, int storage) {
     op->nB = static_cast<int64_t>(itemsB.size());
     op->groups = upload(groups);
     op->nG = static_cast<int64_t>(groups.size());
-    op->lgroups = upload(lgroups);
-    op->nLG = static_cast<int64_t>(lgroups.size());
     if (std::getenv("HMX_VERBOSE"))
         std::fprintf(stderr, "[hmx] storage %d device build: plan %.2f s, total %.2f s\n", storage,
                      t_plan, since());
@@ -631,14 +699,13 @@ size_t scratch_stream_limit() {
 
 void free_scratch(Scratch& sc) {
     for (auto& w : sc.w)
-        for (void* p : {w.S, w.P, w.LP, w.Yp})
+        for (void* p : {w.S, w.P, w.LP})
             if (p) HIPCHECK(hipFree(p));
     sc = Scratch{};
 }
 
 // Per-stream scratch of one pass width, allocated on the stream's first call:
-// the size is checked before anything is allocated, and the four arrays are
-// kept only when all of them were allocated.
+// the size is checked before anything is allocated, and the arrays are kept only when all of them were allocated.
 ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     const size_t sb = static_cast<size_t>(staging(op, W).bytes);
     std::lock_guard<std::mutex> g(op.mu);
@@ -660,15 +727,13 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     if (!s.S) {
         ScratchW n;
         const size_t pb = std::max<int64_t>(op.npartial, 1) * W * p_elem(op.storage);
-        const size_t lb = std::max<int64_t>(op.nlpartial, 1) * W * p_elem(op.storage);
-        const size_t yb = std::max<int64_t>(op.m, 1) * W * p_elem(op.storage);
+        const size_t lb = std::max<int64_t>(op.nlrows, 1) * W * p_elem(op.storage);
         try {
             HIPCHECK(hipMalloc(&n.S, sb));
             HIPCHECK(hipMalloc(&n.P, pb));
             HIPCHECK(hipMalloc(&n.LP, lb));
-            HIPCHECK(hipMalloc(&n.Yp, yb));
         } catch (...) {
-            for (void* p : {n.S, n.P, n.LP, n.Yp})
+            for (void* p : {n.S, n.P, n.LP})
                 if (p) (void)hipFree(p);
             throw;
         }
@@ -677,7 +742,7 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
         // overwrite rows that the first product has already written.
         zero_staging_tail(n.S, staging(op, W), stream);
         s = n;
-        it->second.bytes += sb + pb + lb + yb;
+        it->second.bytes += sb + pb + lb;
         if (std::getenv("HMX_VERBOSE"))
             std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p (%zu bytes), partials %p\n",
                          op.storage, W, s.S, sb, s.P);
@@ -693,9 +758,10 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
     one.colidx = op.colidx;
     one.S = sc.S;
     one.partial = sc.P;
-    one.lpartial = sc.LP;
-    one.Yp = sc.Yp;
-    one.inv_tmap = op.inv_tmap;
+    one.lrows = sc.LP;
+    one.rowsrc = op.rowsrc;
+    one.direct = op.direct;
+    one.io64 = std::is_same<TIO, double>::value;
     one.m = op.m;
     one.tmap0 = op.tmap0;
     one.inv_smap = op.inv_smap;
@@ -715,12 +781,10 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
     A.nG = op.nG;
     A.itemsB = op.itemsB;
     A.nB = op.nB;
-    A.lgroups = op.lgroups;
-    A.nLG = op.nLG;
     A.gather_n = op.n;
     A.gather_insts = 1;
     A.wide = wide_staging(lay);
-    A.out_m = op.m;
+    A.out_m = op.direct ? 0 : op.m;
     for (int rhs0 = 0; rhs0 < nrhs; rhs0 += W) {
         one.rhs0 = rhs0;
         launch_stages<TS, W, TIO, false>(A, one, nullptr, st, &op);
@@ -803,23 +867,6 @@ void* noalloc_base(int device) {
     return g_noalloc_base[device];
 }
 
-// Byte offsets of the four scratch arrays of one pass width inside `scratch`
-// (each 256-byte aligned): S rows, far-field partials, leaf-piece partials, Yp.
-struct NoAllocPlan {
-    size_t s = 0, p = 0, lp = 0, yp = 0, total = 0;
-};
-NoAllocPlan noalloc_plan(const DeviceOp& op, int W) {
-    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t pe = p_elem(op.storage);
-    NoAllocPlan pl;
-    pl.s = 0;
-    pl.p = up(static_cast<size_t>(staging(op, W).bytes));
-    pl.lp = pl.p + up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe);
-    pl.yp = pl.lp + up(static_cast<size_t>(std::max<int64_t>(op.nlpartial, 1)) * W * pe);
-    pl.total = pl.yp + up(static_cast<size_t>(std::max<int64_t>(op.m, 1)) * W * pe);
-    return pl;
-}
-
 template <typename TS, int W, typename TIO>
 void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs,
                  hipStream_t st, unsigned char* base, const NoAllocPlan& pl) {
@@ -828,9 +875,10 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
     one.colidx = op.colidx;
     one.S = base + pl.s;
     one.partial = base + pl.p;
-    one.lpartial = base + pl.lp;
-    one.Yp = base + pl.yp;
-    one.inv_tmap = op.inv_tmap;
+    one.lrows = base + pl.lp;
+    one.rowsrc = op.rowsrc;
+    one.direct = op.direct;
+    one.io64 = std::is_same<TIO, double>::value;
     one.m = op.m;
     one.tmap0 = op.tmap0;
     one.inv_smap = op.inv_smap;
@@ -851,12 +899,10 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
     A.nG = op.nG;
     A.itemsB = op.itemsB;
     A.nB = op.nB;
-    A.lgroups = op.lgroups;
-    A.nLG = op.nLG;
     A.gather_n = op.n;
     A.gather_insts = 1;
     A.wide = wide_staging(lay);
-    A.out_m = op.m;
+    A.out_m = op.direct ? 0 : op.m;
     for (int rhs0 = 0; rhs0 < nrhs; rhs0 += W) {
         one.rhs0 = rhs0;
         launch_stages<TS, W, TIO, false>(A, one, nullptr, st, nullptr);
@@ -966,7 +1012,7 @@ int64_t device_release_scratch(HMatrix& h, void* stream, bool all_streams) {
             // the stream's products may still be running
             HIPCHECK(hipStreamSynchronize(static_cast<hipStream_t>(it->first)));
             for (auto& w : it->second.w)
-                for (void* p : {w.S, w.P, w.LP, w.Yp})
+                for (void* p : {w.S, w.P, w.LP})
                     if (p) freed++;
             free_scratch(it->second);
             it = d->scratch.erase(it);

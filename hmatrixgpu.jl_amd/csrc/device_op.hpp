@@ -9,14 +9,13 @@ namespace hmx {
 struct ScratchW {
     void* S = nullptr;  // (s0 + n + R + 1 + TK) x W source rows (staging_layout)
     void* P = nullptr;   // far-field partial rows x W
-    void* LP = nullptr;  // leaf-piece partial rows x W
-    void* Yp = nullptr;  // leaf results in permuted target order, m x W
+    void* LP = nullptr;  // leaf-result rows x W
 };
 
 struct Scratch {
     ScratchW w[3];  // W = 1, 4, 16
     uint64_t last_use = 0;  // DeviceOp::use_clock at the stream's last product
-    size_t bytes = 0;       // bytes held by the four arrays of every width
+    size_t bytes = 0;       // bytes held by the arrays of every width
 };
 
 inline int w_slot(int W) { return W == 1 ? 0 : W == 4 ? 1 : 2; }
@@ -36,17 +35,15 @@ struct DeviceOp {
     ReduceGroup* groups = nullptr;
     int64_t nG = 0;
     int64_t npartial = 0;
-    LeafGroup* lgroups = nullptr;
-    int64_t nLG = 0;
-    int64_t nlpartial = 0;
+    int64_t nlrows = 0;         // leaf-result rows of one pass
+    RowSrc* rowsrc = nullptr;   // per original target row
+    bool direct = false;        // the leaf kernel writes Y (no item is cut, few rows)
     int32_t* tmap0 = nullptr;
-    int32_t* inv_tmap = nullptr;
     int32_t* inv_smap = nullptr;
     // host copies of the work lists (the batched operator re-packs them)
     std::vector<PairItem> hItemsB;
     std::vector<FarItem> hItemsA;
     std::vector<ReduceGroup> hGroups;
-    std::vector<LeafGroup> hLGroups;
     std::mutex mu;
     std::map<void*, Scratch> scratch;
     uint64_t use_clock = 0;
@@ -98,11 +95,9 @@ struct StageArrays {
     int64_t nG = 0;
     const PairItem* itemsB = nullptr;
     int64_t nB = 0;
-    const LeafGroup* lgroups = nullptr;
-    int64_t nLG = 0;
     int64_t gather_n = 0;   // largest source size over the instances
     int gather_insts = 1;   // instances (grid.y of the gather and the unpermute)
-    int64_t out_m = 0;      // largest target size over the instances
+    int64_t out_m = 0;      // largest target size over the instances that need k_finish
     bool wide = false;      // an instance's S has 4 GiB or more: 64-bit S loads
 };
 // S of 4 GiB or more: beyond the reach of 32-bit buffer offsets
@@ -129,10 +124,9 @@ struct StageTimer {
 };
 
 // The stages of a product pass: gather X -> S, far-field panels (V*X),
-// partial reduce, leaf panels -> permuted rows (or leaf-piece partials), the
-// sum of the leaf pieces, and the unpermute into Y.  The piece sum and the
-// unpermute are timed with the far-field partial reduce (stage 2), so stage 3
-// is the leaf kernel alone.
+// partial reduce, leaf panels -> leaf-result rows, and their piece sums into Y
+// (k_finish, timed with the far-field partial reduce as stage 2, so that
+// stage 3 is the leaf kernel alone).
 template <typename TS, int W, typename TIO, bool BATCH>
 void launch_stages(const StageArrays& A, const InstDesc& one, const InstDesc* insts,
                    hipStream_t st, DeviceOp* prof) {
@@ -165,13 +159,13 @@ void launch_stages(const StageArrays& A, const InstDesc& one, const InstDesc* in
             hipLaunchKernelGGL((k_leaf<TS, W, kPanelPolicy, BATCH, false>), dim3(A.nB),
                                dim3(kWaves * 64), 0, st, A.itemsB, one, insts);
     }
-    StageTimer t(prof, st, 2);
-    if (A.nLG)
-        hipLaunchKernelGGL((k_leaf_reduce<TS, W, BATCH>), dim3(A.nLG), dim3(256), 0, st,
-                           A.lgroups, one, insts);
-    hipLaunchKernelGGL((k_unpermute<TS, W, TIO, BATCH>),
-                       dim3(static_cast<unsigned>((A.out_m + 255) / 256), A.gather_insts),
-                       dim3(256), 0, st, one, insts);
+    if (A.out_m) {
+        StageTimer t(prof, st, 2);
+        constexpr int rows = 256 * kFinCols<W> / W;  // target rows of a workgroup
+        hipLaunchKernelGGL((k_finish<TS, W, TIO, BATCH>),
+                           dim3(static_cast<unsigned>((A.out_m + rows - 1) / rows), A.gather_insts),
+                           dim3(256), 0, st, one, insts);
+    }
 }
 
 // Dispatch order of leaf work items (see device.hip).

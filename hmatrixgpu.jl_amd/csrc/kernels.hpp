@@ -47,30 +47,29 @@ struct Item {
 
 // Leaf work item: one or two consecutive row groups (<= 64 rows each) of the
 // target order.  The columns both row groups need (blocks whose row range
-// covers both) form the shared segment, stored as one panel per row group over
-// the same column indices; the remaining columns of each row group form its
-// private segment.  A single row group (rows[1] == 0) has only a private part.
+// covers both) form the shared segment, over one range of column indices; the
+// remaining columns of each row group form its private segment.  A row group's
+// panel holds its shared and then its private k-tiles back to back, so that one
+// pipeline walks both.  A single row group (rows[1] == 0) has only a private
+// part.
 struct PairItem {
     int64_t out_off[2];  // first permuted target row of each row group
-    int64_t sh_data[2];  // shared-segment panel of each row group
-    int64_t pr_data[2];  // private-segment panel of each row group
+    int64_t data[2];     // panel of each row group: shared, then private k-tiles
     int64_t sh_col;      // colidx offset of the shared columns
     int64_t pr_col[2];   // colidx offset of each private part
     int32_t rows[2];
     int32_t sh_kt;       // k-tiles of the shared segment
     int32_t pr_kt[2];    // k-tiles of each private part
     int32_t inst;        // instance (H-matrix) index in a batched launch
-    int64_t part;        // -1: write Y; else first leaf-partial row of this piece
+    int64_t part;        // first leaf-result row of this item (or k-range piece of one)
 };
 
-// A leaf item cut along k into nparts pieces: the pieces' partial rows
-// (rows[0] + rows[1] each, back to back from pbase) are summed in piece order.
-struct LeafGroup {
-    int64_t pbase;
-    int64_t out_off[2];
-    int32_t rows[2];
-    int32_t nparts;
-    int32_t inst;
+// Where the results of one target row lie: nparts leaf-result rows (one per
+// k-range piece of its leaf item), from `base`, `stride` rows apart.
+struct RowSrc {
+    uint32_t base;
+    int16_t nparts;
+    int16_t stride;
 };
 
 struct ReduceGroup {
@@ -90,9 +89,8 @@ struct InstDesc {
     const int32_t* colidx;
     void* S;                 // source rows from s0: X permuted, then T, then a zero row
     void* partial;           // far-field column-chunk partial sums
-    void* lpartial;          // leaf-piece partial sums
-    void* Yp;                // leaf results in permuted target order (m x W)
-    const int32_t* inv_tmap; // 0-based original target row -> permuted row
+    void* lrows;             // leaf results: rows of W, one set per piece of a leaf item
+    const RowSrc* rowsrc;    // per original target row: its leaf-result rows
     int64_t m;               // target rows
     const int32_t* tmap0;    // permuted target row -> 0-based original row
     const int32_t* inv_smap; // 0-based original source row -> permuted row
@@ -104,7 +102,8 @@ struct InstDesc {
     uint32_t s_rows;         // rows of S (each W elements)
     int32_t nrhs;            // right-hand sides of the call
     int32_t rhs0;            // first right-hand side of this pass
-    int32_t pad;
+    int16_t io64;            // X and Y are FP64 (else FP32)
+    int16_t direct;          // the leaf kernel writes Y itself
 };
 
 // ---- element conversions ---------------------------------------------------
@@ -303,7 +302,9 @@ __device__ inline SRow<T, W> load_srow_wide(const T* S, uint32_t row) {
 
 // One wave's share of a panel: k-tiles kt0, kt0 + kstep, ... of a `rows` x
 // (ktiles * TK) panel at pdata.  B rows come from S: through the column index
-// array (LEAF) or as the contiguous rows col_off + k masked beyond ncols.  The
+// array (LEAF: from colidx + col_off for the first sh_kt k-tiles, from
+// colidx + pr_off for the rest) or as the contiguous rows col_off + k masked
+// beyond ncols.  The
 // accumulated results are handed to emit(row, col, value), row < 64, col < W.
 // W = 16 runs on MFMA (16 right-hand sides as the N dimension); W = 1 and 4 run
 // on the VALU, lane (row li, k-chunk lg).  Loads are issued one k-tile ahead (A
@@ -320,7 +321,8 @@ using PanelAcc = typename std::conditional<
 
 template <typename TS, int W, bool LEAF, int NRT, int CP, bool WIDE>
 __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktiles, int64_t col_off,
-                                            int ncols, const int32_t* colidx,
+                                            int ncols, const int32_t* colidx, int sh_kt,
+                                            int64_t pr_off,
                                             const typename SType<TS, W>::type* S, uint32_t s_rows,
                                             int kt0, int kstep, int lane, float* btile,
                                             PanelAcc<TS, W> (&acc)[NRT]) {
@@ -332,8 +334,10 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     const uint32_t slab = static_cast<uint32_t>(rows) * 64u;
     const __amdgpu_buffer_rsrc_t Ar = make_rsrc(pdata, slab * ktiles);
     const __amdgpu_buffer_rsrc_t Sr = make_rsrc(S, WIDE ? 0u : s_rows * ROWB);
-    const __amdgpu_buffer_rsrc_t Cr =
-        make_rsrc(LEAF ? colidx + col_off : colidx, LEAF ? ktiles * TK * 4 : 0);
+    // Column indices of both segments, addressed by the k-tile of the whole
+    // panel: the private ones from a base moved back by the shared tiles.
+    const int32_t* const csh = colidx + (LEAF ? col_off : 0);
+    const int32_t* const cpr = colidx + (LEAF ? pr_off - static_cast<int64_t>(sh_kt) * TK : 0);
     uint32_t aoff[NRT];
     bool aval[NRT];
 #pragma unroll
@@ -361,6 +365,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     // for the LDS B tile only the column of the row the lane loads (L/4).
     auto load_ix = [&](int kt) {
         IdxV<EPL> r{};
+        const __amdgpu_buffer_rsrc_t Cr = make_rsrc(kt < sh_kt ? csh : cpr, ktiles * TK * 4);
         if constexpr (BLDS) {
             const uint32_t off = static_cast<uint32_t>((kt * TK + (lane >> 2)) * 4);
             r.v[0] = static_cast<int32_t>(__builtin_amdgcn_raw_buffer_load_b32(Cr, off, 0, 0));
@@ -580,8 +585,8 @@ __device__ __forceinline__ void panel_body(const TS* pdata, int rows, int ktiles
     PanelAcc<TS, W> acc[NRT];
 #pragma unroll
     for (int rt = 0; rt < NRT; rt++) acc[rt] = PanelAcc<TS, W>{};
-    panel_accum<TS, W, LEAF, NRT, CP, WIDE>(pdata, rows, ktiles, col_off, ncols, colidx, S, s_rows,
-                                            kt0, kstep, lane, btile, acc);
+    panel_accum<TS, W, LEAF, NRT, CP, WIDE>(pdata, rows, ktiles, col_off, ncols, colidx, 0, 0, S,
+                                            s_rows, kt0, kstep, lane, btile, acc);
     panel_emit<TS, W, NRT>(acc, lane, emit);
 }
 
@@ -605,13 +610,14 @@ __device__ __forceinline__ const InstDesc& inst_of(const InstDesc& one, const In
 }
 
 // Leaf item: for a pair of row groups, waves 0-1 own row group 0 and waves 2-3
-// row group 1; the two waves of a row group split the k-tiles of its shared
-// and then its private panel, keeping one set of accumulators.  Waves 0 and 2
+// row group 1; the two waves of a row group split the k-tiles of its panel (the
+// shared, then the private ones), keeping one set of accumulators and one
+// pipeline: with a pipeline per segment, every piece of an item paid two fills.  Waves 0 and 2
 // (1 and 3) walk the same shared k-tiles at the same time, so each shared B
 // row is fetched once per workgroup and served to the second wave from L1.  A
 // single row group is split over all four waves.  Partial sums are reduced
-// through LDS and written as whole rows, in permuted target order, to Yp (a
-// whole item) or to the leaf-piece partials (a k-range piece of an item).
+// through LDS and written as whole leaf-result rows, which k_finish sums and
+// scatters; the items of a small operator, none of them cut, write Y directly.
 template <typename TS, int W, int CP, bool BATCH, bool WIDE>
 __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict__ items,
                                                       const InstDesc one,
@@ -630,8 +636,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict
     const int kt0 = pair ? (wave & 1) : wave, kstep = pair ? 2 : 4;
     // per-row-group fields by select, not by a runtime index into the item
     const int rows = g ? it.rows[1] : it.rows[0];
-    const int64_t sh_data = g ? it.sh_data[1] : it.sh_data[0];
-    const int64_t pr_data = g ? it.pr_data[1] : it.pr_data[0];
+    const int64_t data = g ? it.data[1] : it.data[0];
     const int64_t pr_col = g ? it.pr_col[1] : it.pr_col[0];
     const int pr_kt = g ? it.pr_kt[1] : it.pr_kt[0];
     __shared__ acc_t red[kWaves][64][W];
@@ -644,16 +649,13 @@ __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict
         PanelAcc<TS, W> acc[NRT];
 #pragma unroll
         for (int rt = 0; rt < NRT; rt++) acc[rt] = PanelAcc<TS, W>{};
-        panel_accum<TS, W, true, NRT, CP, WIDE>(panel + sh_data, rows, it.sh_kt, it.sh_col, 0,
-                                                I.colidx, S, I.s_rows, kt0, kstep, lane,
-                                                btile[wave], acc);
-        panel_accum<TS, W, true, NRT, CP, WIDE>(panel + pr_data, rows, pr_kt, pr_col, 0, I.colidx, S,
-                                                I.s_rows, kt0, kstep, lane, btile[wave], acc);
+        panel_accum<TS, W, true, NRT, CP, WIDE>(panel + data, rows, it.sh_kt + pr_kt, it.sh_col, 0,
+                                                I.colidx, it.sh_kt, pr_col, S, I.s_rows, kt0, kstep,
+                                                lane, btile[wave], acc);
         panel_emit<TS, W, NRT>(acc, lane, emit);
     });
     __syncthreads();
-    acc_t* Yp = static_cast<acc_t*>(I.Yp);
-    acc_t* lpart = static_cast<acc_t*>(I.lpartial);
+    acc_t* lrows = static_cast<acc_t*>(I.lrows);
     const int r0 = it.rows[0], total = r0 + it.rows[1];
     for (int t = threadIdx.x; t < total * W; t += kWaves * 64) {
         const int rr = t / W, j = t % W;
@@ -666,49 +668,61 @@ __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict
 #pragma unroll
             for (int w = 1; w < kWaves; w++) s += red[w][r][j];
         }
-        if (it.part >= 0)
-            lpart[(it.part + rr) * W + j] = s;
-        else
-            Yp[((gg ? it.out_off[1] : it.out_off[0]) + r) * W + j] = s;
+        if (!I.direct) {
+            lrows[(it.part + rr) * W + j] = s;
+        } else if (I.rhs0 + j < I.nrhs) {
+            const int64_t y = I.tmap0[(gg ? it.out_off[1] : it.out_off[0]) + r] +
+                              static_cast<int64_t>(I.rhs0 + j) * I.ldy;
+            if (I.io64)
+                static_cast<double*>(I.Y)[y] = static_cast<double>(s);
+            else
+                static_cast<float*>(I.Y)[y] = static_cast<float>(s);
+        }
     }
 }
 
-// Sum the pieces of a split leaf item in piece order into the permuted rows.
-template <typename TS, int W, bool BATCH>
-__global__ __launch_bounds__(256) void k_leaf_reduce(const LeafGroup* __restrict__ groups,
-                                                     const InstDesc one,
-                                                     const InstDesc* __restrict__ insts) {
-    using acc_t = typename Store<TS>::acc;
-    const LeafGroup g = groups[blockIdx.x];
-    const InstDesc& I = inst_of<BATCH>(one, insts, g.inst);
-    const acc_t* lpart = static_cast<const acc_t*>(I.lpartial);
-    acc_t* Yp = static_cast<acc_t*>(I.Yp);
-    const int r0 = g.rows[0], total = r0 + g.rows[1];
-    for (int t = threadIdx.x; t < total * W; t += blockDim.x) {
-        const int rr = t / W, j = t % W;
-        acc_t s = lpart[(g.pbase + rr) * W + j];
-        for (int p = 1; p < g.nparts; p++)
-            s += lpart[(g.pbase + static_cast<int64_t>(p) * total + rr) * W + j];
-        const int gg = rr < r0 ? 0 : 1, r = rr - gg * r0;
-        Yp[((gg ? g.out_off[1] : g.out_off[0]) + r) * W + j] = s;
-    }
-}
+// Y[i, rhs0 + j] = sum over the pieces of row i, in piece order, for the pass's
+// columns (instance = blockIdx.y).  One thread per original target row and
+// kFinCols<W> columns: the loads of eight pieces are in flight together (the
+// sum itself stays in order), and a wave writes 64 consecutive rows of each
+// column of Y.
+// Bound by the latency of its scattered row reads.  One launch in place of a
+// piece sum with one workgroup per leaf item (128 rows in one workgroup, the
+// pieces in a serial loop) and an unpermute.
+template <int W>
+constexpr int kFinCols = W < 4 ? W : 4;
 
-// Y[i, rhs0 + j] = Yp[inv_tmap[i]][j] for the pass's columns; thread per
-// original target row (instance = blockIdx.y): one whole permuted row read,
-// writes coalesced along each column of Y.
 template <typename TS, int W, typename TIO, bool BATCH>
-__global__ __launch_bounds__(256) void k_unpermute(const InstDesc one,
-                                                   const InstDesc* __restrict__ insts) {
+__global__ __launch_bounds__(256) void k_finish(const InstDesc one,
+                                                const InstDesc* __restrict__ insts) {
     using acc_t = typename Store<TS>::acc;
+    constexpr int C = kFinCols<W>, G = W / C, ROWS = 256 / G;
     const InstDesc& I = inst_of<BATCH>(one, insts, blockIdx.y);
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= I.m) return;
-    const SRowOut<acc_t, W> row = static_cast<const SRowOut<acc_t, W>*>(I.Yp)[I.inv_tmap[i]];
+    if (BATCH && I.direct) return;
+    const int c0 = (threadIdx.x / ROWS) * C;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * ROWS + threadIdx.x % ROWS;
+    if (i >= I.m || I.rhs0 + c0 >= I.nrhs) return;
+    const RowSrc rs = I.rowsrc[i];
+    using row_t = SRowOut<acc_t, C>;
+    const row_t* src = static_cast<const row_t*>(I.lrows) + static_cast<int64_t>(rs.base) * G + c0 / C;
+    const int64_t step = static_cast<int64_t>(rs.stride) * G;
+    row_t s = src[0];
+    for (int p = 1; p < rs.nparts; p += 8) {
+        row_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (p + u < rs.nparts) v[u] = src[(p + u) * step];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (p + u < rs.nparts)
+#pragma unroll
+                for (int j = 0; j < C; j++) s.v[j] += v[u].v[j];
+    }
     TIO* Y = static_cast<TIO*>(I.Y);
 #pragma unroll
-    for (int j = 0; j < W; j++)
-        if (I.rhs0 + j < I.nrhs) Y[i + static_cast<int64_t>(I.rhs0 + j) * I.ldy] = static_cast<TIO>(row.v[j]);
+    for (int j = 0; j < C; j++)
+        if (I.rhs0 + c0 + j < I.nrhs)
+            Y[i + static_cast<int64_t>(I.rhs0 + c0 + j) * I.ldy] = static_cast<TIO>(s.v[j]);
 }
 
 // Far-field work item: up to kWaves consecutive 64-row groups of the stacked V
