@@ -86,7 +86,7 @@ ScratchW& batch_scratch(Batch& b, size_t i, int W) {
     ScratchW& s = v[i];
     if (!s.S) {
         const DeviceOp& op = *b.ops[i];
-        const size_t sb = static_cast<size_t>(staging(op, W).bytes);
+        const size_t sb = static_cast<size_t>(staging(op, W).zero_end);
         HIPCHECK(hipMalloc(&s.S, sb));
         zero_staging_tail(s.S, staging(op, W), nullptr);
         HIPCHECK(hipMalloc(&s.P, std::max<int64_t>(op.npartial, 1) * W * p_elem(op.storage)));

@@ -546,6 +546,7 @@ int hmx_hmatrix_scratch_usage(const hmx_hmatrix* hm, int64_t* bytes, int64_t* en
 int hmx_staging_layout(int64_t n, int64_t R, int32_t storage, int32_t width, int64_t* rows,
                        int64_t* bytes, int64_t* zero_begin, int64_t* zero_end) {
     return guarded([&] {
+        need(width <= 16, "hmx_staging_layout: width must be 1, 4 or 16");
         const hmx::StagingLayout L = hmx::staging_layout(n, R, storage, width);
         if (rows) *rows = L.rows;
         if (bytes) *bytes = L.bytes;

@@ -707,7 +707,7 @@ void free_scratch(Scratch& sc) {
 // Per-stream scratch of one pass width, allocated on the stream's first call:
 // the size is checked before anything is allocated, and the arrays are kept only when all of them were allocated.
 ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
-    const size_t sb = static_cast<size_t>(staging(op, W).bytes);
+    const size_t sb = static_cast<size_t>(staging(op, W).zero_end);
     std::lock_guard<std::mutex> g(op.mu);
     auto it = op.scratch.find(static_cast<void*>(stream));
     if (it == op.scratch.end()) {
@@ -792,14 +792,52 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
     HIPCHECK(hipGetLastError());
 }
 
-// RHS width of a pass: one column -> VALU GEMV, up to 4 -> VALU 4-wide,
-// more -> MFMA 16-wide passes.
+// RHS width of a pass: one column -> VALU GEMV, up to 4 -> VALU 4-wide, more ->
+// MFMA passes of 16, 32 or 48 columns.  A pass reads the whole matrix, so the
+// fewest passes of at most 48 columns are taken, and of those the narrowest that
+// hold nrhs.  At N = 16,384 a pass of 16 / 32 / 48 takes 325 / 376 / 444 us (FP64),
+// 176 / 213 / 264 us (FP32) and 118 / 148 / 178 us (BF16): every wider pass beats the
+// narrow ones that it stands for, from 17 columns on (FP64 with 17: 376 against 560).
+int pass_width(int nrhs) {
+    if (nrhs <= 4) return nrhs == 1 ? 1 : 4;
+    const int passes = (nrhs + 47) / 48;
+    return 16 * ((nrhs + 16 * passes - 1) / (16 * passes));
+}
+
+// Whether a wide pass (32 or 48 columns) can have its scratch: it holds up to three
+// times that of 16 columns.  A stream that is being captured gets no new scratch, and
+// without the memory the product runs in 16-column passes (the same bits).
+bool wide_scratch(DeviceOp& op, hipStream_t st, int W) {
+    {
+        std::lock_guard<std::mutex> g(op.mu);
+        auto it = op.scratch.find(static_cast<void*>(st));
+        if (it != op.scratch.end() && it->second.w[w_slot(W)].S) return true;
+    }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    try {
+        get_scratch(op, st, W);
+        return true;
+    } catch (const Error&) {
+        (void)hipGetLastError();
+        return false;
+    }
+}
+
 template <typename TS, typename TIO>
 void run_w(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs, hipStream_t st) {
-    if (nrhs == 1)
+    const int W = pass_width(nrhs);
+    if (W == 1)
         run<TS, 1, TIO>(op, X, ldx, Y, ldy, nrhs, st);
-    else if (nrhs <= 4)
+    else if (W == 4)
         run<TS, 4, TIO>(op, X, ldx, Y, ldy, nrhs, st);
+    else if (W == 48 && wide_scratch(op, st, 48))
+        run<TS, 48, TIO>(op, X, ldx, Y, ldy, nrhs, st);
+    else if (W == 32 && wide_scratch(op, st, 32))
+        run<TS, 32, TIO>(op, X, ldx, Y, ldy, nrhs, st);
     else
         run<TS, 16, TIO>(op, X, ldx, Y, ldy, nrhs, st);
 }
@@ -913,7 +951,8 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
 template <typename TS, typename TIO>
 void noalloc_w(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs,
                hipStream_t st, size_t limit) {
-    const int W = nrhs == 1 ? 1 : nrhs <= 4 ? 4 : 16;
+    int W = pass_width(nrhs);
+    if (W > 16 && noalloc_plan(op, W).total > limit) W = 16;
     const NoAllocPlan pl = noalloc_plan(op, W);
     if (pl.total > limit)
         throw Error(HMX_ERR_UNSUPPORTED,
@@ -925,6 +964,10 @@ void noalloc_w(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, i
         run_noalloc<TS, 1, TIO>(op, X, ldx, Y, ldy, nrhs, st, base, pl);
     else if (W == 4)
         run_noalloc<TS, 4, TIO>(op, X, ldx, Y, ldy, nrhs, st, base, pl);
+    else if (W == 48)
+        run_noalloc<TS, 48, TIO>(op, X, ldx, Y, ldy, nrhs, st, base, pl);
+    else if (W == 32)
+        run_noalloc<TS, 32, TIO>(op, X, ldx, Y, ldy, nrhs, st, base, pl);
     else
         run_noalloc<TS, 16, TIO>(op, X, ldx, Y, ldy, nrhs, st, base, pl);
 }

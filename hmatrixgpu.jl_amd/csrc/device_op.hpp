@@ -13,12 +13,12 @@ struct ScratchW {
 };
 
 struct Scratch {
-    ScratchW w[3];  // W = 1, 4, 16
+    ScratchW w[5];  // W = 1, 4, 16, 32, 48
     uint64_t last_use = 0;  // DeviceOp::use_clock at the stream's last product
     size_t bytes = 0;       // bytes held by the arrays of every width
 };
 
-inline int w_slot(int W) { return W == 1 ? 0 : W == 4 ? 1 : 2; }
+inline int w_slot(int W) { return W == 1 ? 0 : W == 4 ? 1 : 1 + W / 16; }
 
 struct DeviceOp {
     int storage = 0, device = 0;
@@ -161,9 +161,9 @@ void launch_stages(const StageArrays& A, const InstDesc& one, const InstDesc* in
     }
     if (A.out_m) {
         StageTimer t(prof, st, 2);
-        constexpr int rows = 256 * kFinCols<W> / W;  // target rows of a workgroup
+        constexpr int rows = kFinRows<W>;
         hipLaunchKernelGGL((k_finish<TS, W, TIO, BATCH>),
-                           dim3(static_cast<unsigned>((A.out_m + rows - 1) / rows), A.gather_insts),
+                           dim3(static_cast<unsigned>((A.out_m + rows - 1) / rows), A.gather_insts, kSlices<W>),
                            dim3(256), 0, st, one, insts);
     }
 }

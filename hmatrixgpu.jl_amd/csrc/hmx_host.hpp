@@ -294,7 +294,7 @@ constexpr int kRankFeatures = HMX_RANK_FEATURES;
 inline size_t elem_size(int storage) { return storage == HMX_F64 ? 8 : storage == HMX_F32 ? 4 : 2; }
 inline int tk_of(int storage) { return static_cast<int>(64 / elem_size(storage)); }
 inline size_t s_elem(int storage, int W) {
-    return storage == HMX_F64 ? 8 : (W == 16 && storage == HMX_BF16 ? 2 : 4);
+    return storage == HMX_F64 ? 8 : (W >= 16 && storage == HMX_BF16 ? 2 : 4);
 }
 // The staging array S of one pass: rows n + R + 1 + TK (X permuted, T = V X,
 // a zero row, one k-tile of padding rows), each W elements.  Rows are 32-bit
@@ -307,7 +307,7 @@ struct StagingLayout {
 };
 inline StagingLayout staging_layout(int64_t n, int64_t R, int storage, int W) {
     if (n < 0 || R < 0 || (storage != HMX_F64 && storage != HMX_F32 && storage != HMX_BF16) ||
-        (W != 1 && W != 4 && W != 16))
+        (W != 1 && W != 4 && W != 16 && W != 32 && W != 48))
         throw Error(HMX_ERR_ARG, "staging layout: bad argument");
     StagingLayout L;
     L.rows = n + R + 1 + tk_of(storage);

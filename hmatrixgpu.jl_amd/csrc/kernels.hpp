@@ -153,23 +153,16 @@ struct Store<bf16s> {
     static constexpr int TK = 32, EPL = 8;
     using acc = float;
 };
-// B-operand (S) element type: W = 16 columns -> MFMA operand type; W = 1, 4 (VALU
-// paths) -> the accumulation type
+// Right-hand sides of a pass: 1 or 4 run on the VALU, multiples of 16 on MFMA as
+// kSlices<W> 16-column slices that share each load of the matrix.
+template <int W>
+constexpr bool kMfma = W >= 16;
+template <int W>
+constexpr int kSlices = W >= 16 ? W / 16 : 1;
+// B-operand (S) element type: MFMA -> its operand type; VALU -> the accumulation type
 template <typename TS, int W>
 struct SType {
-    using type = typename Store<TS>::acc;
-};
-template <>
-struct SType<double, 16> {
-    using type = double;
-};
-template <>
-struct SType<float, 16> {
-    using type = float;
-};
-template <>
-struct SType<bf16s, 16> {
-    using type = bf16s;
+    using type = typename std::conditional<kMfma<W>, TS, typename Store<TS>::acc>::type;
 };
 
 constexpr int kWaves = 4;  // waves per workgroup in the panel kernels
@@ -181,9 +174,15 @@ constexpr int kPipe = 3;   // k-tiles in flight per wave (panel_accum)
 // with four); the FP32 16-RHS leaf kernel five (184 VGPRs, 2 waves per SIMD:
 // 0.5% faster than four at 156 VGPRs, 3 waves per SIMD, and the same as six or
 // seven); and the FP32 and FP64 16-RHS far kernels four (0.5% faster).
+// Two and three slices keep three.  The panel kernels ask for two waves per SIMD:
+// the compiler then keeps the accumulators in VGPRs instead of copying them to and
+// from AGPRs, and the FP64 kernels with three slices fit (215 registers against
+// 280; N = 16,384 with 48 right-hand sides 506 -> 444 us; two k-tiles in flight
+// instead: 481 us).
 template <typename TS, bool LEAF, int W>
 constexpr int pipe_depth() {
     if (!LEAF && std::is_same<TS, bf16s>::value) return 2;
+    if (W > 16) return kPipe;
     if (LEAF && W == 16 && std::is_same<TS, float>::value) return 5;
     if (LEAF && W != 4) return 4;
     if (!LEAF && W == 16) return 4;
@@ -314,7 +313,7 @@ __device__ inline SRow<T, W> load_srow_wide(const T* S, uint32_t row) {
 // or per-lane partial sums (W = 1, 4).
 template <typename TS, int W>
 using PanelAcc = typename std::conditional<
-    W == 16,
+    kMfma<W>,
     typename std::conditional<std::is_same<typename Store<TS>::acc, double>::value, f64x4,
                               f32x4>::type,
     SRow<typename Store<TS>::acc, W>>::type;
@@ -325,7 +324,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                                             int64_t pr_off,
                                             const typename SType<TS, W>::type* S, uint32_t s_rows,
                                             int kt0, int kstep, int lane, float* btile,
-                                            PanelAcc<TS, W> (&acc)[NRT]) {
+                                            PanelAcc<TS, W>* acc) {
     using acc_t = typename Store<TS>::acc;
     using s_t = typename SType<TS, W>::type;
     constexpr int TK = Store<TS>::TK, EPL = Store<TS>::EPL;
@@ -346,8 +345,9 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
         aval[rt] = li < rr;
         aoff[rt] = static_cast<uint32_t>((16 * rt * TK + (rr * lg + li) * EPL) * sizeof(TS));
     }
-    const uint32_t bcol = (W == 16 ? li : 0) * SB;
-    using brow_t = typename std::conditional<W == 16, s_t, SRow<s_t, W>>::type;
+    constexpr int NB = kSlices<W>;
+    const uint32_t bcol = (kMfma<W> ? li : 0) * SB;
+    using brow_t = typename std::conditional<kMfma<W>, s_t, SRow<s_t, W>>::type;
 
     // FP32 with 16 RHS: the k-tile's B rows (16 rows x 64 B = 1 KB) arrive as
     // one 16-byte load per lane (lane L: row L/4, bytes 16 (L%4) of it, with
@@ -355,11 +355,12 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     // to the MFMA operand layout through the wave's LDS tile btile (rows padded
     // to kBTileStride floats, so that the four lane groups read distinct
     // banks).  One load instruction per k-tile instead of EPL.
-    constexpr bool BLDS = std::is_same<TS, float>::value && W == 16;
+    // With more slices, one such load and one pass through the tile per slice.
+    constexpr bool BLDS = std::is_same<TS, float>::value && kMfma<W>;
     struct Stage {
         u32x4 a[NRT];
-        brow_t b[EPL];
-        u32x4 bq;
+        brow_t b[NB][EPL];
+        u32x4 bq[NB];
     };
     // Column indices of k-tile kt: the lane's EPL columns (lane group lg), or
     // for the LDS B tile only the column of the row the lane loads (L/4).
@@ -396,11 +397,15 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                 ok = k < ncols;
                 row = ok ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
             }
-            if constexpr (WIDE) {
-                st.bq = *reinterpret_cast<const u32x4*>(S + static_cast<uint64_t>(row) * 16 + (lane & 3) * 4);
-            } else {
-                const uint32_t o = ok ? row * ROWB + (lane & 3) * 16 : kOOB;
-                st.bq = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(Sr, o, 0, 0));
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                if constexpr (WIDE) {
+                    st.bq[b] = *reinterpret_cast<const u32x4*>(S + static_cast<uint64_t>(row) * W +
+                                                               16 * b + (lane & 3) * 4);
+                } else {
+                    const uint32_t o = ok ? row * ROWB + 64 * b + (lane & 3) * 16 : kOOB;
+                    st.bq[b] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(Sr, o, 0, 0));
+                }
             }
             return st;
         }
@@ -414,10 +419,12 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                     const int k = kt * TK + lg * EPL + e;
                     row = k < ncols ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
                 }
-                if constexpr (W == 16)
-                    st.b[e] = S[static_cast<uint64_t>(row) * 16 + li];
-                else
-                    st.b[e] = load_srow_wide<s_t, W>(S, row);
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    if constexpr (kMfma<W>)
+                        st.b[b][e] = S[static_cast<uint64_t>(row) * W + 16 * b + li];
+                    else
+                        st.b[b][e] = load_srow_wide<s_t, W>(S, row);
             } else {
                 uint32_t o;
                 if constexpr (LEAF) {
@@ -426,49 +433,62 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                     const int k = kt * TK + lg * EPL + e;
                     o = k < ncols ? static_cast<uint32_t>(col_off + k) * ROWB + bcol : kOOB;
                 }
-                if constexpr (W == 16)
-                    st.b[e] = buf_load<s_t>(Sr, o);
-                else
-                    st.b[e] = load_srow<s_t, W>(Sr, o);
+#pragma unroll
+                for (int b = 0; b < NB; b++)  // a masked column (kOOB) stays out of range for every slice
+                    if constexpr (kMfma<W>)
+                        st.b[b][e] = buf_load<s_t>(Sr, o == kOOB ? kOOB : o + 16 * b * SB);
+                    else
+                        st.b[b][e] = load_srow<s_t, W>(Sr, o);
             }
         }
         return st;
     };
 
     auto compute = [&](const Stage& st) {
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        float bv[NB][4] = {};
         if constexpr (BLDS) {
             // LDS operations of one wave complete in order: the reads see this
-            // write, and the next k-tile's write follows these reads.  The wave
-            // barriers keep the compiler from moving them across each other.
-            *reinterpret_cast<u32x4*>(btile + (lane >> 2) * kBTileStride + (lane & 3) * 4) = st.bq;
-            __builtin_amdgcn_wave_barrier();
+            // write, and the next write follows these reads.  The wave barriers
+            // keep the compiler from moving them across each other.
 #pragma unroll
-            for (int e = 0; e < 4; e++) bv[e] = btile[(lg * 4 + e) * kBTileStride + li];
-            __builtin_amdgcn_wave_barrier();
+            for (int b = 0; b < NB; b++) {
+                *reinterpret_cast<u32x4*>(btile + (lane >> 2) * kBTileStride + (lane & 3) * 4) = st.bq[b];
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int e = 0; e < 4; e++) bv[b][e] = btile[(lg * 4 + e) * kBTileStride + li];
+                __builtin_amdgcn_wave_barrier();
+            }
         }
 #pragma unroll
         for (int rt = 0; rt < NRT; rt++) {
             const u32x4 raw = st.a[rt];
-            if constexpr (W == 16) {
+            PanelAcc<TS, W>* const c = acc + rt * NB;  // the slices' accumulators of this row tile
+            if constexpr (kMfma<W>) {
                 if constexpr (BLDS) {
                     f32x4 a = __builtin_bit_cast(f32x4, raw);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bv[0], acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, bv[1], acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, bv[2], acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, bv[3], acc[rt], 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int b = 0; b < NB; b++)
+                            c[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], bv[b][e], c[b], 0, 0, 0);
                 } else if constexpr (std::is_same<TS, double>::value) {
                     typedef double d2 __attribute__((ext_vector_type(2)));
                     d2 a = __builtin_bit_cast(d2, raw);
-                    acc[rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, st.b[0], acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, st.b[1], acc[rt], 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 2; e++)
+#pragma unroll
+                        for (int b = 0; b < NB; b++)
+                            c[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], st.b[b][e], c[b], 0, 0, 0);
                 } else {
                     bf16x8 a = __builtin_bit_cast(bf16x8, raw);
-                    uint16_t bb[8];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) bb[e] = st.b[e].u;
-                    bf16x8 bv = __builtin_bit_cast(bf16x8, bb);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[rt], 0, 0, 0);
+                    for (int b = 0; b < NB; b++) {
+                        uint16_t bb[8];
+#pragma unroll
+                        for (int e = 0; e < 8; e++) bb[e] = st.b[b][e].u;
+                        bf16x8 bx = __builtin_bit_cast(bf16x8, bb);
+                        c[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bx, c[b], 0, 0, 0);
+                    }
                 }
             } else {
                 acc_t av[EPL];
@@ -489,7 +509,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                 for (int w = 0; w < W; w++) {
                     acc_t s = acc[rt].v[w];
 #pragma unroll
-                    for (int e = 0; e < EPL; e++) s += av[e] * st.b[e].v[w];
+                    for (int e = 0; e < EPL; e++) s += av[e] * st.b[0][e].v[w];
                     acc[rt].v[w] = s;
                 }
             }
@@ -548,24 +568,25 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
         if (j < rem) compute(st[j]);
 }
 
-// Hand the accumulated tile results to emit(row, col, value), row < 16*NRT.
-template <typename TS, int W, int NRT, typename Emit>
-__device__ __forceinline__ void panel_emit(PanelAcc<TS, W> (&acc)[NRT], int lane, Emit&& emit) {
+// Hand the accumulated results of slice b (VALU: of all columns) to
+// emit(row, col, value), row < 16*nrt, col < min(W, 16).
+template <typename TS, int W, typename Emit>
+__device__ __forceinline__ void panel_emit(const PanelAcc<TS, W>* acc, int nrt, int b, int lane,
+                                           Emit&& emit) {
     using acc_t = typename Store<TS>::acc;
     const int li = lane & 15, lg = lane >> 4;
-    if constexpr (W == 16) {
-        // MFMA 16x16 output, column li: f32 accumulators hold rows 4*lg+v of the
-        // row tile, the f64 instruction holds rows 4*v+lg.
 #pragma unroll
-        for (int rt = 0; rt < NRT; rt++)
+    for (int rt = 0; rt < 4; rt++) {
+        if (rt >= nrt) break;
+        if constexpr (kMfma<W>) {
+            // MFMA 16x16 output, column li: f32 accumulators hold rows 4*lg+v of the
+            // row tile, the f64 instruction holds rows 4*v+lg.
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = std::is_same<TS, double>::value ? 4 * v + lg : 4 * lg + v;
-                emit(16 * rt + row, li, static_cast<acc_t>(acc[rt][v]));
+                emit(16 * rt + row, li, static_cast<acc_t>(acc[rt * kSlices<W> + b][v]));
             }
-    } else {
-#pragma unroll
-        for (int rt = 0; rt < NRT; rt++)
+        } else {
 #pragma unroll
             for (int w = 0; w < W; w++) {
                 acc_t v = acc[rt].v[w];
@@ -573,21 +594,8 @@ __device__ __forceinline__ void panel_emit(PanelAcc<TS, W> (&acc)[NRT], int lane
                 v += __shfl_xor(v, 32);
                 if (lg == 0) emit(16 * rt + li, w, v);
             }
+        }
     }
-}
-
-// One wave's share of a panel, accumulated from zero and emitted.
-template <typename TS, int W, bool LEAF, int NRT, int CP, bool WIDE, typename Emit>
-__device__ __forceinline__ void panel_body(const TS* pdata, int rows, int ktiles, int64_t col_off,
-                                           int ncols, const int32_t* colidx,
-                                           const typename SType<TS, W>::type* S, uint32_t s_rows,
-                                           int kt0, int kstep, int lane, float* btile, Emit&& emit) {
-    PanelAcc<TS, W> acc[NRT];
-#pragma unroll
-    for (int rt = 0; rt < NRT; rt++) acc[rt] = PanelAcc<TS, W>{};
-    panel_accum<TS, W, LEAF, NRT, CP, WIDE>(pdata, rows, ktiles, col_off, ncols, colidx, 0, 0, S,
-                                            s_rows, kt0, kstep, lane, btile, acc);
-    panel_emit<TS, W, NRT>(acc, lane, emit);
 }
 
 template <typename F>
@@ -619,7 +627,7 @@ __device__ __forceinline__ const InstDesc& inst_of(const InstDesc& one, const In
 // through LDS and written as whole leaf-result rows, which k_finish sums and
 // scatters; the items of a small operator, none of them cut, write Y directly.
 template <typename TS, int W, int CP, bool BATCH, bool WIDE>
-__global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict__ items,
+__global__ __launch_bounds__(kWaves * 64, 2) void k_leaf(const PairItem* __restrict__ items,
                                                       const InstDesc one,
                                                       const InstDesc* __restrict__ insts) {
     using acc_t = typename Store<TS>::acc;
@@ -639,51 +647,56 @@ __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict
     const int64_t data = g ? it.data[1] : it.data[0];
     const int64_t pr_col = g ? it.pr_col[1] : it.pr_col[0];
     const int pr_kt = g ? it.pr_kt[1] : it.pr_kt[0];
-    __shared__ acc_t red[kWaves][64][W];
-    __shared__ float btile[kWaves][16 * kBTileStride];  // B tiles (FP32, 16 RHS only)
-    auto emit = [&](int row, int j, acc_t v) { red[wave][row][j] = v; };
+    constexpr int NB = kSlices<W>, WS = W / NB;  // columns of a slice
+    __shared__ acc_t red[kWaves][64][WS];
+    __shared__ float btile[kWaves][16 * kBTileStride];  // B tiles (FP32 on MFMA only)
     const TS* panel = static_cast<const TS*>(I.panel);
     const s_t* S = static_cast<const s_t*>(I.S);
+    PanelAcc<TS, W> acc[4 * NB];
+#pragma unroll
+    for (int q = 0; q < 4 * NB; q++) acc[q] = PanelAcc<TS, W>{};
     dispatch_nrt(rows, [&](auto nrt) {
         constexpr int NRT = decltype(nrt)::value;
-        PanelAcc<TS, W> acc[NRT];
-#pragma unroll
-        for (int rt = 0; rt < NRT; rt++) acc[rt] = PanelAcc<TS, W>{};
         panel_accum<TS, W, true, NRT, CP, WIDE>(panel + data, rows, it.sh_kt + pr_kt, it.sh_col, 0,
                                                 I.colidx, it.sh_kt, pr_col, S, I.s_rows, kt0, kstep,
                                                 lane, btile[wave], acc);
-        panel_emit<TS, W, NRT>(acc, lane, emit);
     });
-    __syncthreads();
     acc_t* lrows = static_cast<acc_t*>(I.lrows);
     const int r0 = it.rows[0], total = r0 + it.rows[1];
-    for (int t = threadIdx.x; t < total * W; t += kWaves * 64) {
-        const int rr = t / W, j = t % W;
-        const int gg = rr < r0 ? 0 : 1, r = rr - gg * r0;
-        acc_t s;
-        if (pair) {
-            s = red[2 * gg][r][j] + red[2 * gg + 1][r][j];
-        } else {
-            s = red[0][r][j];
 #pragma unroll
-            for (int w = 1; w < kWaves; w++) s += red[w][r][j];
-        }
-        if (!I.direct) {
-            lrows[(it.part + rr) * W + j] = s;
-        } else if (I.rhs0 + j < I.nrhs) {
-            const int64_t y = I.tmap0[(gg ? it.out_off[1] : it.out_off[0]) + r] +
-                              static_cast<int64_t>(I.rhs0 + j) * I.ldy;
-            if (I.io64)
-                static_cast<double*>(I.Y)[y] = static_cast<double>(s);
-            else
-                static_cast<float*>(I.Y)[y] = static_cast<float>(s);
+    for (int b = 0; b < NB; b++) {  // one slice at a time through LDS
+        if (b) __syncthreads();
+        panel_emit<TS, W>(acc, (rows + 15) >> 4, b, lane,
+                          [&](int row, int j, acc_t v) { red[wave][row][j] = v; });
+        __syncthreads();
+        for (int t = threadIdx.x; t < total * WS; t += kWaves * 64) {
+            const int rr = t / WS, j = t % WS, c = b * WS + j;
+            const int gg = rr < r0 ? 0 : 1, r = rr - gg * r0;
+            acc_t s;
+            if (pair) {
+                s = red[2 * gg][r][j] + red[2 * gg + 1][r][j];
+            } else {
+                s = red[0][r][j];
+#pragma unroll
+                for (int w = 1; w < kWaves; w++) s += red[w][r][j];
+            }
+            if (!I.direct) {
+                lrows[(it.part + rr) * W + c] = s;
+            } else if (I.rhs0 + c < I.nrhs) {
+                const int64_t y = I.tmap0[(gg ? it.out_off[1] : it.out_off[0]) + r] +
+                                  static_cast<int64_t>(I.rhs0 + c) * I.ldy;
+                if (I.io64)
+                    static_cast<double*>(I.Y)[y] = static_cast<double>(s);
+                else
+                    static_cast<float*>(I.Y)[y] = static_cast<float>(s);
+            }
         }
     }
 }
 
 // Y[i, rhs0 + j] = sum over the pieces of row i, in piece order, for the pass's
-// columns (instance = blockIdx.y).  One thread per original target row and
-// kFinCols<W> columns: the loads of eight pieces are in flight together (the
+// columns (instance = blockIdx.y, slice = blockIdx.z).  One thread per original
+// target row and kFinCols<W> columns: the loads of eight pieces are in flight together (the
 // sum itself stays in order), and a wave writes 64 consecutive rows of each
 // column of Y.
 // Bound by the latency of its scattered row reads.  One launch in place of a
@@ -691,15 +704,17 @@ __global__ __launch_bounds__(kWaves * 64) void k_leaf(const PairItem* __restrict
 // pieces in a serial loop) and an unpermute.
 template <int W>
 constexpr int kFinCols = W < 4 ? W : 4;
+template <int W>
+constexpr int kFinRows = kMfma<W> ? 64 : 256;  // target rows of a workgroup
 
 template <typename TS, int W, typename TIO, bool BATCH>
 __global__ __launch_bounds__(256) void k_finish(const InstDesc one,
                                                 const InstDesc* __restrict__ insts) {
     using acc_t = typename Store<TS>::acc;
-    constexpr int C = kFinCols<W>, G = W / C, ROWS = 256 / G;
+    constexpr int C = kFinCols<W>, G = W / C, ROWS = kFinRows<W>;
     const InstDesc& I = inst_of<BATCH>(one, insts, blockIdx.y);
     if (BATCH && I.direct) return;
-    const int c0 = (threadIdx.x / ROWS) * C;
+    const int c0 = (threadIdx.x / ROWS) * C + 16 * blockIdx.z;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * ROWS + threadIdx.x % ROWS;
     if (i >= I.m || I.rhs0 + c0 >= I.nrhs) return;
     const RowSrc rs = I.rowsrc[i];
@@ -744,7 +759,7 @@ struct FarItem {
 };
 
 template <typename TS, int W, int CP, bool BATCH, bool WIDE>
-__global__ __launch_bounds__(kWaves * 64) void k_far(const FarItem* __restrict__ items,
+__global__ __launch_bounds__(kWaves * 64, 2) void k_far(const FarItem* __restrict__ items,
                                                      const InstDesc one,
                                                      const InstDesc* __restrict__ insts) {
     using acc_t = typename Store<TS>::acc;
@@ -762,18 +777,25 @@ __global__ __launch_bounds__(kWaves * 64) void k_far(const FarItem* __restrict__
     const int64_t orow = it.out_off + 64 * wave;
     s_t* S = static_cast<s_t*>(I.S);
     acc_t* partial = static_cast<acc_t*>(I.partial);
-    auto emit = [&](int row, int j, acc_t v) {
-        if (row >= rows) return;
-        if (it.to_T)
-            S[(I.s0 + I.n + orow + row) * W + j] = from_double<s_t>(static_cast<double>(v));
-        else
-            partial[(orow + row) * W + j] = v;
-    };
+    constexpr int NB = kSlices<W>;
+    PanelAcc<TS, W> acc[4 * NB];
+#pragma unroll
+    for (int q = 0; q < 4 * NB; q++) acc[q] = PanelAcc<TS, W>{};
     dispatch_nrt(rows, [&](auto nrt) {
-        panel_body<TS, W, false, decltype(nrt)::value, CP, WIDE>(pd, rows, it.ktiles, it.col_off,
-                                                                 it.ncols, nullptr, S, I.s_rows, 0,
-                                                                 1, lane, btile[wave], emit);
+        panel_accum<TS, W, false, decltype(nrt)::value, CP, WIDE>(
+            pd, rows, it.ktiles, it.col_off, it.ncols, nullptr, 0, 0, S, I.s_rows, 0, 1, lane,
+            btile[wave], acc);
     });
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        panel_emit<TS, W>(acc, (rows + 15) >> 4, b, lane, [&](int row, int j, acc_t v) {
+            if (row >= rows) return;
+            const int c = 16 * b + j;
+            if (it.to_T)
+                S[(I.s0 + I.n + orow + row) * W + c] = from_double<s_t>(static_cast<double>(v));
+            else
+                partial[(orow + row) * W + c] = v;
+        });
 }
 
 // Sum the column-chunk partials of far-field row groups in a fixed order.

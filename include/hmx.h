@@ -248,8 +248,9 @@ int hmx_hmatrix_release_scratch(hmx_hmatrix* h, void* stream, int32_t all_stream
  * it.  No reference counterpart (monitoring of the scratch above). */
 int hmx_hmatrix_scratch_usage(const hmx_hmatrix* h, int64_t* bytes, int64_t* entries);
 /* Size of the source/T staging array that one product pass of `width`
- * right-hand sides (1, 4 or 16; the product runs ceil(nrhs / 16) passes of 16
- * for nrhs > 4) allocates for an operator of `storage` precision with n source
+ * right-hand sides (1, 4 or 16; a product with nrhs > 16 runs ceil(nrhs / 48)
+ * passes of 16, 32 or 48, the wider ones with two or three times the bytes of 16,
+ * or passes of 16 where that memory is not to be had) allocates for an operator of `storage` precision with n source
  * rows and R stacked low-rank rows (sizes[4] of hmx_hmatrix_sizes): *rows rows
  * of *bytes / *rows bytes, of which [*zero_begin, *zero_end) must read zero
  * (cleared at allocation, and by hmx_matvec_noalloc on every call).  The
@@ -314,7 +315,8 @@ int hmx_hmatrix_destroy(hmx_hmatrix* h);
  * and stream-ordered on `stream` (NULL = default stream).  Scratch is per
  * (H-matrix, stream), so concurrent calls on different streams are safe;
  * concurrent calls on one stream are ordered by the stream.  The first call on
- * a new stream allocates its scratch (hipMalloc). */
+ * a new stream allocates its scratch (hipMalloc), and so does the first with a
+ * wider pass (nrhs 1, 2-4, 5-16, 17-32 and 33 or more differ). */
 int hmx_matvec(hmx_hmatrix* h, int32_t storage, const void* X, int64_t ldx, void* Y, int64_t ldy,
                int32_t nrhs, int32_t io_dtype, void* stream);
 
