@@ -337,6 +337,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     // panel: the private ones from a base moved back by the shared tiles.
     const int32_t* const csh = colidx + (LEAF ? col_off : 0);
     const int32_t* const cpr = colidx + (LEAF ? pr_off - static_cast<int64_t>(sh_kt) * TK : 0);
+    const __amdgpu_buffer_rsrc_t Csh = make_rsrc(csh, ktiles * TK * 4), Cpr = make_rsrc(cpr, ktiles * TK * 4);
     uint32_t aoff[NRT];
     bool aval[NRT];
 #pragma unroll
@@ -366,7 +367,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     // for the LDS B tile only the column of the row the lane loads (L/4).
     auto load_ix = [&](int kt) {
         IdxV<EPL> r{};
-        const __amdgpu_buffer_rsrc_t Cr = make_rsrc(kt < sh_kt ? csh : cpr, ktiles * TK * 4);
+        const __amdgpu_buffer_rsrc_t Cr = kt < sh_kt ? Csh : Cpr;
         if constexpr (BLDS) {
             const uint32_t off = static_cast<uint32_t>((kt * TK + (lane >> 2)) * 4);
             r.v[0] = static_cast<int32_t>(__builtin_amdgcn_raw_buffer_load_b32(Cr, off, 0, 0));
