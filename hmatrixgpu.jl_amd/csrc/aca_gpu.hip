@@ -24,6 +24,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <future>
+#include <iterator>
+#include <numeric>
 
 namespace hmx {
 
@@ -369,16 +371,24 @@ __device__ __forceinline__ void wave_apply_q(int m, int k, const double* A, cons
 }
 
 // R_U R_V' -> one-sided Jacobi SVD -> sorted singular values, W, Z2 and the
-// truncation rank.  M and Z (k x k) live in LDS when they fit (kLdsK) and in
-// the block's global scratch otherwise; the arithmetic and its order are the
-// same either way.
-constexpr int kLdsK = 32;
+// truncation rank.  M and Z (k x k) live in LDS up to k = kLdsK and in the block's
+// global scratch beyond; the arithmetic and its order are the same either way.
+// In LDS a column has an odd stride, so that the lanes of a round, each in
+// another column, read distinct banks (an even one put all 16 pairs of k = 32 on
+// one bank).  The LDS of a launch is sized by its k class (kRecClass).  Cores of
+// k > 32 used to rotate in global memory: of the 79,786 blocks at N = 32,768 (tol
+// 1e-6) the 17,815 of k > 32 took 116 of the 150 ms of the kernel, and now 31.
+constexpr int kLdsK = 64;
+constexpr int kRecClass[] = {32, 40, kLdsK};
+__host__ __device__ constexpr int rec_stride(int k) { return k | 1; }
+constexpr size_t rec_lds_bytes(int k) { return size_t(2) * k * rec_stride(k) * sizeof(double); }
 
 template <bool IN_LDS>
 __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const double* QV, double* M,
                                         double* Z, double* W, double* Z2, double* nrm, double* sig,
                                         double* ord, int m, int n, int k, double eps, int lane) {
 #pragma clang fp contract(off)
+    const int ld = IN_LDS ? rec_stride(k) : k;  // column stride of M and Z
     for (int idx = lane; idx < k * k; idx += 64) {  // (R_U R_V')[i, j]
         const int i = idx % k, j = idx / k;
         double s = 0.0;
@@ -386,8 +396,8 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
             const double pr = QU[i + static_cast<int64_t>(l) * m] * QV[j + static_cast<int64_t>(l) * n];
             s = s + pr;
         }
-        M[i + j * k] = s;
-        Z[idx] = i == j ? 1.0 : 0.0;
+        M[i + j * ld] = s;
+        Z[i + j * ld] = i == j ? 1.0 : 0.0;
     }
     __syncthreads();
     // one-sided Jacobi, round-robin sweeps: the k'/2 disjoint pairs of a round
@@ -396,9 +406,11 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
     const double tol = 2.220446049250313e-16;
     const int kp = k + (k & 1);
     if constexpr (IN_LDS) {
-        // k <= 32, so at most 16 pairs: the pair's lane forms the three sums in
-        // order (as the host does) and its rotation; four lanes per pair then
-        // apply it, each to every fourth element (elementwise, so the same bits)
+        // At most 32 pairs: the pair's lane forms the three sums in order (as the
+        // host does) and its rotation; four lanes per pair (two beyond 16 pairs)
+        // then apply it, each to its share of the elements (elementwise, so the
+        // same bits).
+        const int per = kp / 2 <= 16 ? 4 : 2;
         __shared__ double rot_c[kLdsK / 2], rot_s[kLdsK / 2];
         __shared__ int rot_pq[kLdsK / 2];
         for (int sweep = 0; sweep < 80; sweep++) {
@@ -411,9 +423,10 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
                     const int p = min(a, b), q = max(a, b);
                     int code = -1;
                     if (q < k) {
-                        const double* ap = M + p * k;
-                        const double* aq = M + q * k;
+                        const double* ap = M + p * ld;
+                        const double* aq = M + q * ld;
                         double al = 0.0, be = 0.0, ga = 0.0;
+#pragma unroll 4
                         for (int i = 0; i < k; i++) {
                             const double x = ap[i], y = aq[i];
                             const double xx = x * x, yy = y * y, xy = x * y;
@@ -435,15 +448,15 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
                     rot_pq[pi] = code;
                 }
                 __syncthreads();
-                const int pi = lane >> 2, part = lane & 3;
+                const int pi = lane / per, part = lane % per;
                 if (pi < kp / 2 && rot_pq[pi] >= 0) {
                     const int p = rot_pq[pi] & 255, q = rot_pq[pi] >> 8;
                     const double c = rot_c[pi], s = rot_s[pi];
-                    double* ap = M + p * k;
-                    double* aq = M + q * k;
-                    double* zp = Z + p * k;
-                    double* zq = Z + q * k;
-                    for (int i = part; i < k; i += 4) {
+                    double* ap = M + p * ld;
+                    double* aq = M + q * ld;
+                    double* zp = Z + p * ld;
+                    double* zq = Z + q * ld;
+                    for (int i = part; i < k; i += per) {
                         const double x = ap[i], y = aq[i];
                         ap[i] = c * x - s * y;
                         aq[i] = s * x + c * y;
@@ -465,8 +478,8 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
                     const int b = 1 + (kp - 2 - pi + rnd) % (kp - 1);
                     const int p = min(a, b), q = max(a, b);
                     if (q >= k) continue;
-                    double* ap = M + p * k;
-                    double* aq = M + q * k;
+                    double* ap = M + p * ld;
+                    double* aq = M + q * ld;
                     double al = 0.0, be = 0.0, ga = 0.0;
                     for (int i = 0; i < k; i++) {
                         const double x = ap[i], y = aq[i];
@@ -482,8 +495,8 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
                         (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
                     const double c = 1.0 / sqrt(1.0 + t * t);
                     const double s = c * t;
-                    double* zp = Z + p * k;
-                    double* zq = Z + q * k;
+                    double* zp = Z + p * ld;
+                    double* zq = Z + q * ld;
                     for (int i = 0; i < k; i++) {
                         const double x = ap[i], y = aq[i];
                         ap[i] = c * x - s * y;
@@ -501,7 +514,7 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
     for (int j = lane; j < k; j += 64) {
         double s = 0.0;
         for (int i = 0; i < k; i++) {
-            const double pr = M[i + j * k] * M[i + j * k];
+            const double pr = M[i + j * ld] * M[i + j * ld];
             s = s + pr;
         }
         nrm[j] = sqrt(s);
@@ -522,8 +535,8 @@ __device__ __forceinline__ void rec_svd(RecTask& T, const double* QU, const doub
     __syncthreads();
     for (int idx = lane; idx < k * k; idx += 64) {
         const int i = idx % k, j = idx / k, o = static_cast<int>(ord[j]);
-        W[i + j * k] = nrm[o] > 0.0 ? M[i + o * k] / nrm[o] : 0.0;
-        Z2[i + j * k] = Z[i + o * k];
+        W[i + j * k] = nrm[o] > 0.0 ? M[i + o * ld] / nrm[o] : 0.0;
+        Z2[i + j * k] = Z[i + o * ld];
     }
     for (int j = lane; j < k; j += 64) sig[j] = nrm[static_cast<int>(ord[j])];
     __syncthreads();
@@ -566,9 +579,9 @@ __global__ __launch_bounds__(64) void k_rec_core(RecTask* __restrict__ tasks, do
     double* tv = tu + k;
     wave_qr(m, k, QU, tu, lane);
     wave_qr(n, k, QV, tv, lane);
-    __shared__ double mz[2 * kLdsK * kLdsK];
+    extern __shared__ double mz[];
     if (k <= kLdsK)
-        rec_svd<true>(T, QU, QV, mz, mz + k * k, W, Z2, nrm, sig, ord, m, n, k, eps, lane);
+        rec_svd<true>(T, QU, QV, mz, mz + k * rec_stride(k), W, Z2, nrm, sig, ord, m, n, k, eps, lane);
     else
         rec_svd<false>(T, QU, QV, M, Z, W, Z2, nrm, sig, ord, m, n, k, eps, lane);
 }
@@ -696,6 +709,9 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
     try {
         HIPCHECK(hipEventCreate(&e0));
         HIPCHECK(hipEventCreate(&e1));
+        HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_rec_core),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     static_cast<int>(rec_lds_bytes(kLdsK))));
         const int64_t nb = static_cast<int64_t>(blocks.size());
         // most expensive first: cost ~ (m + n) * cap^2
         auto cost = [&](int64_t b) {
@@ -818,15 +834,44 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
                     sc += need;
                     f1++;
                 }
+                // by k class, so that each launch reserves the LDS its blocks need:
+                // beyond kLdsK first (the longest), then the largest class down
+                auto k_class = [](int32_t k) {
+                    int c = 0;
+                    for (int lim : kRecClass) c += k > lim;
+                    return c;
+                };
+                std::vector<size_t> ord(rt.size());
+                std::iota(ord.begin(), ord.end(), size_t(0));
+                std::stable_sort(ord.begin(), ord.end(), [&](size_t a, size_t b) {
+                    return k_class(rt[a].k) > k_class(rt[b].k);
+                });
+                {
+                    std::vector<RecTask> rs(rt.size());
+                    std::vector<int64_t> is(rt.size());
+                    for (size_t q = 0; q < ord.size(); q++) {
+                        rs[q] = rt[ord[q]];
+                        is[q] = ids[ord[q]];
+                    }
+                    rt.swap(rs);
+                    ids.swap(is);
+                }
                 double* dscr = nullptr;
                 HIPCHECK(hipMalloc(&dscr, std::max<int64_t>(sc, 1) * sizeof(double)));
                 owned.push_back(dscr);
                 RecTask* drt = upload(rt);
                 owned.push_back(drt);
                 HIPCHECK(hipEventRecord(e0, nullptr));
-                hipLaunchKernelGGL(k_rec_core, dim3(rt.size()), dim3(64), 0, nullptr, drt, pool, dscr,
-                                   svd_eps);
-                HIPCHECK(hipGetLastError());
+                for (size_t q0 = 0; q0 < rt.size();) {
+                    const int c = k_class(rt[q0].k);
+                    size_t q1 = q0;
+                    while (q1 < rt.size() && k_class(rt[q1].k) == c) q1++;
+                    const size_t lds = c < int(std::size(kRecClass)) ? rec_lds_bytes(kRecClass[c]) : 0;
+                    hipLaunchKernelGGL(k_rec_core, dim3(q1 - q0), dim3(64), lds, nullptr, drt + q0,
+                                       pool, dscr, svd_eps);
+                    HIPCHECK(hipGetLastError());
+                    q0 = q1;
+                }
                 HIPCHECK(hipMemcpy(rt.data(), drt, rt.size() * sizeof(RecTask), hipMemcpyDeviceToHost));
                 std::vector<Out> outs;
                 int64_t otot = 0;
