@@ -600,18 +600,18 @@ __global__ __launch_bounds__(64) void k_rec_apply(const RecTask* __restrict__ ta
     const double* tu = sig + 2 * k;
     const double* tv = tu + k;
     double* U = out + T.ooff;                        // m x r, column-major
-    double* V = U + static_cast<int64_t>(m) * r;     // r x n, column-major: (j, c) at j + c*r
+    double* V = U + static_cast<int64_t>(m) * r;     // r x n, row-major: (j, c) at j*n + c
     for (int64_t idx = lane; idx < static_cast<int64_t>(m) * r; idx += 64) {
         const int i = static_cast<int>(idx % m), j = static_cast<int>(idx / m);
         U[idx] = i < k ? W[i + j * k] * sig[j] : 0.0;
     }
     for (int64_t idx = lane; idx < static_cast<int64_t>(n) * r; idx += 64) {
         const int i = static_cast<int>(idx % n), j = static_cast<int>(idx / n);  // C(i, j)
-        V[j + static_cast<int64_t>(i) * r] = i < k ? Z2[i + j * k] : 0.0;
+        V[idx] = i < k ? Z2[i + j * k] : 0.0;
     }
     __syncthreads();
     wave_apply_q(m, k, pool + T.uoff, tu, r, U, m, 1, lane);
-    wave_apply_q(n, k, pool + T.voff, tv, r, V, 1, r, lane);
+    wave_apply_q(n, k, pool + T.voff, tv, r, V, n, 1, lane);
 }
 
 int64_t round_cap(int64_t c, int64_t kmax) {
@@ -625,7 +625,7 @@ int64_t aca_round_cap(int64_t c, int64_t kmax) { return round_cap(c, kmax); }
 
 void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<int32_t> caps,
              double eps, double svd_eps, int nthreads, AcaStats* stats, const AcaDone& on_done,
-             const std::vector<int64_t>& probe, const AcaRefine& refine) {
+             const AcaSlabDone& on_slab, const std::vector<int64_t>& probe, const AcaRefine& refine) {
     // The 1/r kernel and the dipole tensor: their entries (subtractions,
     // products, sqrt, division) are correctly rounded on both sides, so the
     // device reproduces the host factors exactly; the log kernel's device log()
@@ -682,7 +682,8 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
     hipEvent_t e0 = nullptr, e1 = nullptr;
     // Host side of finished blocks: their terms are packed on the device,
     // copied into one of two pinned staging buffers and handed to a worker that
-    // transposes V and calls on_done (recompression) on nthreads threads while
+    // copies recompressed factors into slabs (on_slab), or transposes V and calls
+    // on_done (recompression on the host), on nthreads threads while
     // the GPU proceeds with the next pass or chunk.
     struct Staging {
         double* host = nullptr;
@@ -738,8 +739,7 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
         std::vector<int64_t> seen_ids;
         std::vector<int32_t> seen_ranks;
         // Hand finished blocks to the host: copy `tot` doubles at dsrc into a
-        // pinned staging buffer, then a worker builds the LowRank of every entry
-        // of `outs` and calls on_done.
+        // pinned staging buffer, then a worker hands on the entries of `outs`.
         struct Out {
             int64_t block, m, n, k, aca_k, off;
         };
@@ -759,8 +759,41 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
             if (tot > 0)
                 HIPCHECK(hipMemcpy(st.host, dsrc, tot * sizeof(double), hipMemcpyDeviceToHost));
             const double* hbuf = st.host;
-            st.job = std::async(std::launch::async, [outs = std::move(outs), hbuf, nthreads,
-                                                     recompressed, &on_done] {
+            if (recompressed) {
+                // consecutive blocks share a slab; at least a few slabs per thread
+                const int64_t lim = std::min(kSlabBytes / 8, std::max<int64_t>(
+                                                                 1 << 15, tot / (4 * std::max(1, nthreads))));
+                std::vector<std::pair<size_t, size_t>> cuts;
+                for (size_t a = 0; a < outs.size();) {
+                    size_t b = a;
+                    int64_t len = 0;
+                    while (b < outs.size() && (b == a || len + outs[b].k * (outs[b].m + outs[b].n) <= lim)) {
+                        len += outs[b].k * (outs[b].m + outs[b].n);
+                        b++;
+                    }
+                    cuts.push_back({a, b});
+                    a = b;
+                }
+                st.job = std::async(std::launch::async, [outs = std::move(outs), cuts = std::move(cuts),
+                                                         hbuf, nthreads, &on_slab] {
+                    parallel_for(static_cast<int64_t>(cuts.size()), nthreads, [&](int64_t c) {
+                        auto s = std::make_unique<FactorSlab>();
+                        const int64_t base = outs[cuts[c].first].off;
+                        int64_t len = 0;
+                        for (size_t q = cuts[c].first; q < cuts[c].second; q++) {
+                            const Out& o = outs[q];
+                            s->parts.push_back({o.block, o.aca_k, o.m, o.n, o.k, o.off - base});
+                            len = o.off - base + o.k * (o.m + o.n);
+                        }
+                        s->data.resize(static_cast<size_t>(len));
+                        advise_huge_pages(s->data.data(), static_cast<size_t>(len) * sizeof(double));
+                        if (len) std::memcpy(s->data.data(), hbuf + base, static_cast<size_t>(len) * sizeof(double));
+                        on_slab(std::move(s));
+                    });
+                });
+                return;
+            }
+            st.job = std::async(std::launch::async, [outs = std::move(outs), hbuf, nthreads, &on_done] {
                 parallel_for(static_cast<int64_t>(outs.size()), nthreads, [&](int64_t f) {
                     const Out& o = outs[f];
                     LowRank L;
@@ -769,14 +802,10 @@ void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<
                     L.k = o.k;
                     L.U.assign(hbuf + o.off, hbuf + o.off + o.k * o.m);
                     const double* src = hbuf + o.off + o.k * o.m;
-                    if (recompressed) {  // V already k x n column-major
-                        L.V.assign(src, src + o.k * o.n);
-                    } else {             // terms q: V row q contiguous over n
-                        L.V.resize(static_cast<size_t>(o.k * o.n));
-                        for (int64_t q = 0; q < o.k; q++)
-                            for (int64_t j = 0; j < o.n; j++) L.V[q + j * o.k] = src[q * o.n + j];
-                    }
-                    on_done(o.block, o.aca_k, std::move(L), recompressed);
+                    L.V.resize(static_cast<size_t>(o.k * o.n));  // terms q: V row q contiguous over n
+                    for (int64_t q = 0; q < o.k; q++)
+                        for (int64_t j = 0; j < o.n; j++) L.V[q + j * o.k] = src[q * o.n + j];
+                    on_done(o.block, o.aca_k, std::move(L));
                 });
             });
         };

@@ -262,13 +262,26 @@ struct AcaStats {
 // refine(ids, aca_ranks, caps) may rewrite the capacities of the other blocks.
 using AcaRefine = std::function<void(const std::vector<int64_t>&, const std::vector<int32_t>&,
                                      std::vector<int32_t>&)>;
-// on_done(block, aca_rank, factors, recompressed): factors are the ACA+ terms,
-// or (svd_eps >= 0) their device recompression at svd_eps (bit-identical to
-// svd_recompress).
-using AcaDone = std::function<void(int64_t, int64_t, LowRank&&, bool)>;
+// svd_eps < 0: on_done(block, aca_rank, factors) receives the ACA+ terms of every
+// block.  svd_eps >= 0: on_slab receives their device recompression at svd_eps
+// (bit-identical to svd_recompress) instead.
+using AcaDone = std::function<void(int64_t, int64_t, LowRank&&)>;
+// Recompressed factors of many blocks in one buffer: per part U (m x k column-major)
+// at off, then V (k x n, row-major).  One buffer of up to kSlabBytes instead of two
+// vectors per block: its pages are faulted 2 MiB at a time (the factors of N = 32,768,
+// 2.5 GB, took 0.36 s to place into fresh per-block vectors).
+struct FactorSlab {
+    struct Part {
+        int64_t block, aca_k, m, n, k, off;
+    };
+    Payload data;
+    std::vector<Part> parts;
+};
+constexpr int64_t kSlabBytes = int64_t(16) << 20;
+using AcaSlabDone = std::function<void(std::unique_ptr<FactorSlab>)>;
 void gpu_aca(const HMatrix& h, const std::vector<AcaBlock>& blocks, std::vector<int32_t> caps,
              double eps, double svd_eps, int nthreads, AcaStats* stats, const AcaDone& on_done,
-             const std::vector<int64_t>& probe = {}, const AcaRefine& refine = nullptr);
+             const AcaSlabDone& on_slab, const std::vector<int64_t>& probe = {}, const AcaRefine& refine = nullptr);
 // capacity rounding of a pass (multiple of 4, at least 4, at most kmax)
 int64_t aca_round_cap(int64_t c, int64_t kmax);
 

@@ -296,6 +296,9 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
                            h->approx_stats[b].feat);
     }
     std::vector<LowRank> lr(approx.size());
+    std::vector<std::unique_ptr<FactorSlab>> slabs;  // recompressed on the GPU (lr stays empty)
+    std::mutex slab_mu;
+    std::vector<int64_t> rank(approx.size(), 0);
     if (opt->aca_device == 1) {
         // batched ACA+ on the GPU with a rank capacity per block; recompression
         // on host threads as blocks come back
@@ -363,9 +366,18 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
         }
         h->device = opt->device;
         gpu_aca(*h, blocks, caps, eps / 10.0, svd ? eps : -1.0, threads, opt->stats,
-                [&](int64_t b, int64_t aca_k, LowRank&& f, bool recompressed) {
+                [&](int64_t b, int64_t aca_k, LowRank&& f) {
                     h->approx_stats[b].aca_rank = static_cast<int32_t>(aca_k);
-                    lr[b] = (svd && !recompressed) ? svd_recompress(f, eps) : std::move(f);
+                    lr[b] = svd ? svd_recompress(f, eps) : std::move(f);
+                    rank[b] = lr[b].k;
+                },
+                [&](std::unique_ptr<FactorSlab> s) {
+                    for (const FactorSlab::Part& p : s->parts) {
+                        h->approx_stats[p.block].aca_rank = static_cast<int32_t>(p.aca_k);
+                        rank[p.block] = p.k;
+                    }
+                    std::lock_guard<std::mutex> g(slab_mu);
+                    slabs.push_back(std::move(s));
                 },
                 probe, refine);
     } else
@@ -391,9 +403,10 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
         LowRank f = aca_plus(mm, nn, rowf, colf, eps / 10.0, 0);  // hmatrix.jl:194-196
         h->approx_stats[b].aca_rank = static_cast<int32_t>(f.k);
         if (svd) f = svd_recompress(f, eps);                       // :197-199
+        rank[b] = f.k;
         lr[b] = std::move(f);
     });
-    for (int64_t b = 0; b < na; b++) h->approx_stats[b].rank = static_cast<int32_t>(lr[b].k);
+    for (int64_t b = 0; b < na; b++) h->approx_stats[b].rank = static_cast<int32_t>(rank[b]);
 
     // Storage test (m+n)k < mn, else the block is stored dense after all direct
     // blocks, in approx order (hmatrix.jl:202-213).
@@ -409,7 +422,7 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
     for (size_t b = 0; b < approx.size(); b++) {
         const ClusterNode& a = T.nodes[approx[b].first];
         const ClusterNode& s = S.nodes[approx[b].second];
-        const int64_t mm = a.end - a.start, nn = s.end - s.start, k = lr[b].k;
+        const int64_t mm = a.end - a.start, nn = s.end - s.start, k = rank[b];
         if (mm * k + k * nn < mm * nn) {
             LowRankBlock L{a.start, a.end - 1, s.start, s.end - 1, k, ulen, vlen, vx,
                            approx[b].second};
@@ -429,7 +442,23 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
     h->V.resize(static_cast<size_t>(vlen));
     advise_huge_pages(h->U.data(), h->U.size() * sizeof(double));
     advise_huge_pages(h->V.data(), h->V.size() * sizeof(double));
-    parallel_for(static_cast<int64_t>(keep.size()), threads, [&](int64_t q) {
+    std::vector<int64_t> pos(slabs.empty() ? 0 : approx.size(), -1);  // block -> h->lowrank
+    if (!slabs.empty())
+        for (size_t q = 0; q < keep.size(); q++) pos[keep[q]] = static_cast<int64_t>(q);
+    parallel_for(static_cast<int64_t>(slabs.size()), threads, [&](int64_t s) {
+        const FactorSlab& S = *slabs[s];
+        for (const FactorSlab::Part& p : S.parts) {
+            if (pos[p.block] < 0) continue;  // stored dense
+            const LowRankBlock& L = h->lowrank[pos[p.block]];
+            const double* src = S.data.data() + p.off;
+            double* U = h->U.data() + L.uoff;  // vec(U'): U row-major m x k
+            for (int64_t i = 0; i < p.m; i++)
+                for (int64_t c = 0; c < p.k; c++) U[i * p.k + c] = src[i + c * p.m];
+            std::copy(src + p.k * p.m, src + p.k * (p.m + p.n), h->V.data() + L.voff);
+        }
+        slabs[s].reset();
+    });
+    parallel_for(slabs.empty() ? static_cast<int64_t>(keep.size()) : 0, threads, [&](int64_t q) {
         LowRank& f = lr[keep[q]];
         const LowRankBlock& L = h->lowrank[q];
         double* U = h->U.data() + L.uoff;  // vec(U'): U row-major m x k
