@@ -167,28 +167,50 @@ struct SType {
 
 constexpr int kWaves = 4;  // waves per workgroup in the panel kernels
 constexpr int kPipe = 3;   // k-tiles in flight per wave (panel_accum)
-// Exceptions, each measured on the MI355X: the BF16 far-field kernel keeps two
-// (its panels are a few k-tiles long; 1.5% faster for the BF16 product, slower
-// for FP32 and FP64); the leaf kernels with 1 or 16 right-hand sides four
-// (0.2-0.7% faster for every storage; the 4-wide leaf kernel was 0.7% slower
-// with four); the FP32 16-RHS leaf kernel five (184 VGPRs, 2 waves per SIMD:
-// 0.5% faster than four at 156 VGPRs, 3 waves per SIMD, and the same as six or
-// seven); and the FP32 and FP64 16-RHS far kernels four (0.5% faster).
-// Two and three slices keep three.  The panel kernels ask for two waves per SIMD:
-// the compiler then keeps the accumulators in VGPRs instead of copying them to and
-// from AGPRs, and the FP64 kernels with three slices fit (215 registers against
-// 280; N = 16,384 with 48 right-hand sides 506 -> 444 us; two k-tiles in flight
-// instead: 481 us).
+// Exceptions, each measured on the MI355X with the B tiles in LDS: the BF16 far-field
+// kernel keeps two (its panels are a few k-tiles long); the leaf kernels with one right-hand
+// side and the FP64 ones with 16 keep four (five: FP64 with one 1% faster at N = 50,000 and
+// 7% slower at 4,096); the FP32 and BF16 leaf kernels with 16 keep six (N = 100,000: FP32
+// 2131 -> 2118 us against five, BF16 1090 -> 1082 against four; seven and eight the same
+// or slower); the FP32 and FP64 far kernels with 16 four.  The 4-wide kernels spill from
+// five on (FP32, N = 20,011: 188 -> 263 us).  Two and three slices keep three.  The panel
+// kernels ask for two waves per SIMD: the compiler then keeps the accumulators in VGPRs
+// instead of copying them to and from AGPRs, and the FP64 kernels with three slices fit
+// (N = 16,384 with 48 right-hand sides 506 -> 444 us; two k-tiles in flight instead:
+// 481 us).  Asking for four makes the VALU kernels spill.
 template <typename TS, bool LEAF, int W>
 constexpr int pipe_depth() {
     if (!LEAF && std::is_same<TS, bf16s>::value) return 2;
     if (W > 16) return kPipe;
-    if (LEAF && W == 16 && std::is_same<TS, float>::value) return 5;
+    if (LEAF && W == 16 && !std::is_same<TS, double>::value) return 6;
     if (LEAF && W != 4) return 4;
     if (!LEAF && W == 16) return 4;
     return kPipe;
 }
-constexpr int kBTileStride = 20;  // floats per row of a wave's FP32 B tile in LDS (16 + 4 pad)
+// B tile of one wave and slice: the k-tile's TK rows of S, brought in by one load
+// instruction (lane L: LB bytes, chunk L % LPR of row L / LPR) and handed to the lanes
+// that need them through LDS.  STRIDE pads a row so that the lane groups of a read hit
+// distinct banks: FP32 on MFMA 64 + 16 bytes, FP64 128 + 64, BF16 32 + 8; the VALU
+// paths read whole rows, the same one in 16 lanes, and need no padding.  The texture
+// unit's load instructions bound these kernels next to HBM: before, only FP32 on MFMA
+// went this way, and the others loaded every operand for every lane.  us per product,
+// before -> now: N = 20,011 with four right-hand sides FP32 213 -> 188, BF16 163 -> 123,
+// FP64 391 -> 350; with one BF16 114 -> 98; N = 4,096 FP64 with one 45 -> 41;
+// N = 50,000 BF16 with 16 429 -> 410.
+template <typename TS, int W>
+struct BTile {
+    using s_t = typename SType<TS, W>::type;
+    static constexpr int RB = (kMfma<W> ? 16 : W) * static_cast<int>(sizeof(s_t));
+    static constexpr int LB = RB < 16 ? RB : 16, LPR = RB / LB;
+    static constexpr int LANES = Store<TS>::TK * LPR;
+    static constexpr int STRIDE =
+        !kMfma<W> ? RB : std::is_same<TS, float>::value ? 80 : std::is_same<TS, double>::value ? 192 : 40;
+    static constexpr int BYTES = Store<TS>::TK * STRIDE;
+    static_assert(LANES <= 64, "one load per lane");
+    // the lane's part of a row, as loaded
+    using part_t = typename std::conditional<
+        LB == 16, u32x4, typename std::conditional<LB == 8, uint64_t, uint32_t>::type>::type;
+};
 
 // ---- the panel kernel ----------------------------------------------------------
 // Buffer resources (raw, stride 0): loads past num_records return 0, which masks
@@ -206,52 +228,6 @@ __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t by
                                              kRsrcWord3);
 }
 
-template <int N>
-struct IdxV {
-    int32_t v[N];
-};
-
-// Column indices of the lane's EPL columns of k-tile kt.
-template <int EPL, int TK>
-__device__ inline IdxV<EPL> load_idx(__amdgpu_buffer_rsrc_t C, int kt, int lg) {
-    IdxV<EPL> r;
-    const uint32_t off = static_cast<uint32_t>((kt * TK + lg * EPL) * 4);
-    if constexpr (EPL == 2) {
-        auto v = __builtin_amdgcn_raw_buffer_load_b64(C, off, 0, 0);
-        r.v[0] = static_cast<int32_t>(v[0]);
-        r.v[1] = static_cast<int32_t>(v[1]);
-    } else if constexpr (EPL == 4) {
-        auto v = __builtin_amdgcn_raw_buffer_load_b128(C, off, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; e++) r.v[e] = static_cast<int32_t>(v[e]);
-    } else {
-        auto v0 = __builtin_amdgcn_raw_buffer_load_b128(C, off, 0, 0);
-        auto v1 = __builtin_amdgcn_raw_buffer_load_b128(C, off + 16, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            r.v[e] = static_cast<int32_t>(v0[e]);
-            r.v[4 + e] = static_cast<int32_t>(v1[e]);
-        }
-    }
-    return r;
-}
-
-template <typename T>
-__device__ inline T buf_load(__amdgpu_buffer_rsrc_t R, uint32_t off);
-template <>
-__device__ inline double buf_load<double>(__amdgpu_buffer_rsrc_t R, uint32_t off) {
-    auto v = __builtin_amdgcn_raw_buffer_load_b64(R, off, 0, 0);
-    return __builtin_bit_cast(double, v);
-}
-template <>
-__device__ inline float buf_load<float>(__amdgpu_buffer_rsrc_t R, uint32_t off) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(R, off, 0, 0));
-}
-template <>
-__device__ inline bf16s buf_load<bf16s>(__amdgpu_buffer_rsrc_t R, uint32_t off) {
-    return bf16s{__builtin_amdgcn_raw_buffer_load_b16(R, off, 0, 0)};
-}
-
 // One S row of W values for the VALU paths (W = 1 or 4).
 template <typename T, int W>
 struct SRow {
@@ -263,41 +239,6 @@ template <typename T, int W>
 struct alignas(sizeof(T) * W >= 16 ? 16 : sizeof(T) * W) SRowOut {
     T v[W];
 };
-
-template <typename T, int W>
-__device__ inline SRow<T, W> load_srow(__amdgpu_buffer_rsrc_t R, uint32_t off) {
-    SRow<T, W> r;
-    if constexpr (W == 1) {
-        r.v[0] = buf_load<T>(R, off);
-    } else if constexpr (std::is_same<T, float>::value) {
-        auto q = __builtin_amdgcn_raw_buffer_load_b128(R, off, 0, 0);
-        f32x4 f = __builtin_bit_cast(f32x4, q);
-        r.v[0] = f.x; r.v[1] = f.y; r.v[2] = f.z; r.v[3] = f.w;
-    } else {
-        typedef double d2 __attribute__((ext_vector_type(2)));
-        d2 lo = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(R, off, 0, 0));
-        d2 hi = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(R, off + 16, 0, 0));
-        r.v[0] = lo.x; r.v[1] = lo.y; r.v[2] = hi.x; r.v[3] = hi.y;
-    }
-    return r;
-}
-
-// The same loads for an S of 4 GiB or more, which a buffer's 32-bit offsets
-// cannot reach: global loads at 64-bit addresses of row `row`.  Rows are
-// always in range here (a masked column reads the zero padding row instead).
-template <typename T, int W>
-__device__ inline SRow<T, W> load_srow_wide(const T* S, uint32_t row) {
-    const T* p = S + static_cast<uint64_t>(row) * W;
-    SRow<T, W> r;
-    if constexpr (W == 1) {
-        r.v[0] = *p;
-    } else {
-        const SRowOut<T, W> q = *reinterpret_cast<const SRowOut<T, W>*>(p);
-#pragma unroll
-        for (int w = 0; w < W; w++) r.v[w] = q.v[w];
-    }
-    return r;
-}
 
 // One wave's share of a panel: k-tiles kt0, kt0 + kstep, ... of a `rows` x
 // (ktiles * TK) panel at pdata.  B rows come from S: through the column index
@@ -323,7 +264,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                                             int ncols, const int32_t* colidx, int sh_kt,
                                             int64_t pr_off,
                                             const typename SType<TS, W>::type* S, uint32_t s_rows,
-                                            int kt0, int kstep, int lane, float* btile,
+                                            int kt0, int kstep, int lane, char* btile,
                                             PanelAcc<TS, W>* acc) {
     using acc_t = typename Store<TS>::acc;
     using s_t = typename SType<TS, W>::type;
@@ -348,35 +289,26 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     }
     constexpr int NB = kSlices<W>;
     const uint32_t bcol = (kMfma<W> ? li : 0) * SB;
-    using brow_t = typename std::conditional<kMfma<W>, s_t, SRow<s_t, W>>::type;
+    using brow_t = typename std::conditional<kMfma<W>, s_t, SRowOut<s_t, W>>::type;
 
-    // FP32 with 16 RHS: the k-tile's B rows (16 rows x 64 B = 1 KB) arrive as
-    // one 16-byte load per lane (lane L: row L/4, bytes 16 (L%4) of it, with
-    // that column's index loaded by the lane itself) and are redistributed
-    // to the MFMA operand layout through the wave's LDS tile btile (rows padded
-    // to kBTileStride floats, so that the four lane groups read distinct
-    // banks).  One load instruction per k-tile instead of EPL.
-    // With more slices, one such load and one pass through the tile per slice.
-    constexpr bool BLDS = std::is_same<TS, float>::value && kMfma<W>;
+    // The k-tile's B rows arrive as one load per lane and slice (BTile) instead of one
+    // per operand: with four right-hand sides the 16 lanes of a lane group used to load
+    // the same rows, 4 KB for 256 B, and held them in registers for every stage.
+    using BT = BTile<TS, W>;
+    using part_t = typename BT::part_t;
+    const int brow = lane / BT::LPR, bpart = lane % BT::LPR;
+    const bool bact = lane < BT::LANES;
     struct Stage {
         u32x4 a[NRT];
-        brow_t b[NB][EPL];
-        u32x4 bq[NB];
+        part_t b[NB];
     };
-    // Column indices of k-tile kt: the lane's EPL columns (lane group lg), or
-    // for the LDS B tile only the column of the row the lane loads (L/4).
+    // Column index of the row the lane loads.
     auto load_ix = [&](int kt) {
-        IdxV<EPL> r{};
         const __amdgpu_buffer_rsrc_t Cr = kt < sh_kt ? Csh : Cpr;
-        if constexpr (BLDS) {
-            const uint32_t off = static_cast<uint32_t>((kt * TK + (lane >> 2)) * 4);
-            r.v[0] = static_cast<int32_t>(__builtin_amdgcn_raw_buffer_load_b32(Cr, off, 0, 0));
-        } else {
-            r = load_idx<EPL, TK>(Cr, kt, lg);
-        }
-        return r;
+        const uint32_t off = bact ? static_cast<uint32_t>((kt * TK + brow) * 4) : kOOB;
+        return static_cast<int32_t>(__builtin_amdgcn_raw_buffer_load_b32(Cr, off, 0, 0));
     };
-    auto load_stage = [&](int kt, const IdxV<EPL>& ix) {
+    auto load_stage = [&](int kt, int32_t ix) {
         Stage st;
         const uint32_t base = static_cast<uint32_t>(kt) * slab;
         // A far panel's last k-tile is zero-padded past ncols: a lane whose
@@ -388,84 +320,69 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
             const uint32_t o = aval[rt] && kin ? base + aoff[rt] : kOOB;
             st.a[rt] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(Ar, o, 0, CP));
         }
-        if constexpr (BLDS) {
-            uint32_t row;
-            bool ok = true;
-            if constexpr (LEAF) {
-                row = static_cast<uint32_t>(ix.v[0]);
-            } else {
-                const int k = kt * TK + (lane >> 2);
-                ok = k < ncols;
-                row = ok ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
-            }
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                if constexpr (WIDE) {
-                    st.bq[b] = *reinterpret_cast<const u32x4*>(S + static_cast<uint64_t>(row) * W +
-                                                               16 * b + (lane & 3) * 4);
-                } else {
-                    const uint32_t o = ok ? row * ROWB + 64 * b + (lane & 3) * 16 : kOOB;
-                    st.bq[b] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(Sr, o, 0, 0));
-                }
-            }
-            return st;
+        uint32_t row;
+        bool ok = bact;
+        if constexpr (LEAF) {
+            row = static_cast<uint32_t>(ix);
+        } else {
+            const int k = kt * TK + brow;
+            ok = ok && k < ncols;
+            row = ok ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
         }
 #pragma unroll
-        for (int e = 0; e < EPL; e++) {
+        for (int b = 0; b < NB; b++) {
             if constexpr (WIDE) {
-                uint32_t row;
-                if constexpr (LEAF) {
-                    row = static_cast<uint32_t>(ix.v[e]);
-                } else {
-                    const int k = kt * TK + lg * EPL + e;
-                    row = k < ncols ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
-                }
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    if constexpr (kMfma<W>)
-                        st.b[b][e] = S[static_cast<uint64_t>(row) * W + 16 * b + li];
-                    else
-                        st.b[b][e] = load_srow_wide<s_t, W>(S, row);
+                st.b[b] = part_t{};
+                if (bact)
+                    st.b[b] = *reinterpret_cast<const part_t*>(
+                        reinterpret_cast<const char*>(S) + static_cast<uint64_t>(row) * ROWB +
+                        b * BT::RB + bpart * BT::LB);
             } else {
-                uint32_t o;
-                if constexpr (LEAF) {
-                    o = static_cast<uint32_t>(ix.v[e]) * ROWB + bcol;
-                } else {
-                    const int k = kt * TK + lg * EPL + e;
-                    o = k < ncols ? static_cast<uint32_t>(col_off + k) * ROWB + bcol : kOOB;
-                }
-#pragma unroll
-                for (int b = 0; b < NB; b++)  // a masked column (kOOB) stays out of range for every slice
-                    if constexpr (kMfma<W>)
-                        st.b[b][e] = buf_load<s_t>(Sr, o == kOOB ? kOOB : o + 16 * b * SB);
-                    else
-                        st.b[b][e] = load_srow<s_t, W>(Sr, o);
+                const uint32_t o = ok ? row * ROWB + b * BT::RB + bpart * BT::LB : kOOB;
+                if constexpr (BT::LB == 16)
+                    st.b[b] = __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b128(Sr, o, 0, 0));
+                else if constexpr (BT::LB == 8)
+                    st.b[b] = __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b64(Sr, o, 0, 0));
+                else
+                    st.b[b] = __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b32(Sr, o, 0, 0));
             }
         }
         return st;
     };
 
     auto compute = [&](const Stage& st) {
-        float bv[NB][4] = {};
-        if constexpr (BLDS) {
+        // the lane's B operands: column li of rows lg * EPL + e (MFMA), or those rows
+        brow_t bv[NB][EPL];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
             // LDS operations of one wave complete in order: the reads see this
             // write, and the next write follows these reads.  The wave barriers
             // keep the compiler from moving them across each other.
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                *reinterpret_cast<u32x4*>(btile + (lane >> 2) * kBTileStride + (lane & 3) * 4) = st.bq[b];
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int e = 0; e < 4; e++) bv[b][e] = btile[(lg * 4 + e) * kBTileStride + li];
-                __builtin_amdgcn_wave_barrier();
+            if (BT::LANES == 64 || bact) {
+                char* const d = btile + brow * BT::STRIDE + bpart * BT::LB;
+                if constexpr (BT::STRIDE % BT::LB == 0) {
+                    *reinterpret_cast<part_t*>(d) = st.b[b];
+                } else {  // rows aligned to eight bytes only
+                    struct Half {
+                        uint64_t v[2];
+                    };
+                    const Half h = __builtin_bit_cast(Half, st.b[b]);
+                    reinterpret_cast<uint64_t*>(d)[0] = h.v[0];
+                    reinterpret_cast<uint64_t*>(d)[1] = h.v[1];
+                }
             }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int e = 0; e < EPL; e++)
+                bv[b][e] = *reinterpret_cast<const brow_t*>(btile + (lg * EPL + e) * BT::STRIDE + bcol);
+            __builtin_amdgcn_wave_barrier();
         }
 #pragma unroll
         for (int rt = 0; rt < NRT; rt++) {
             const u32x4 raw = st.a[rt];
             PanelAcc<TS, W>* const c = acc + rt * NB;  // the slices' accumulators of this row tile
             if constexpr (kMfma<W>) {
-                if constexpr (BLDS) {
+                if constexpr (std::is_same<TS, float>::value) {
                     f32x4 a = __builtin_bit_cast(f32x4, raw);
 #pragma unroll
                     for (int e = 0; e < 4; e++)
@@ -479,14 +396,14 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                     for (int e = 0; e < 2; e++)
 #pragma unroll
                         for (int b = 0; b < NB; b++)
-                            c[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], st.b[b][e], c[b], 0, 0, 0);
+                            c[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], bv[b][e], c[b], 0, 0, 0);
                 } else {
                     bf16x8 a = __builtin_bit_cast(bf16x8, raw);
 #pragma unroll
                     for (int b = 0; b < NB; b++) {
                         uint16_t bb[8];
 #pragma unroll
-                        for (int e = 0; e < 8; e++) bb[e] = st.b[b][e].u;
+                        for (int e = 0; e < 8; e++) bb[e] = bv[b][e].u;
                         bf16x8 bx = __builtin_bit_cast(bf16x8, bb);
                         c[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bx, c[b], 0, 0, 0);
                     }
@@ -510,7 +427,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
                 for (int w = 0; w < W; w++) {
                     acc_t s = acc[rt].v[w];
 #pragma unroll
-                    for (int e = 0; e < EPL; e++) s += av[e] * st.b[0][e].v[w];
+                    for (int e = 0; e < EPL; e++) s += av[e] * bv[0][e].v[w];
                     acc[rt].v[w] = s;
                 }
             }
@@ -533,7 +450,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     const int mine = kt0 < ktiles ? (ktiles - kt0 + kstep - 1) / kstep : 0;
     constexpr int D = pipe_depth<TS, LEAF, W>();
     int kt = kt0;
-    IdxV<EPL> ix[D];
+    int32_t ix[D];
     Stage st[D];
     // The prologue issues its loads in the loop's own order (indices, then
     // stages, then the next index), fenced against rescheduling: the wait the
@@ -542,7 +459,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     // would make it wait for every load in flight at each iteration.
 #pragma unroll
     for (int d = 0; d < D; d++) {
-        ix[d] = IdxV<EPL>{};
+        ix[d] = 0;
         if constexpr (LEAF) ix[d] = load_ix(kt + d * kstep);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -650,7 +567,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_leaf(const PairItem* __restr
     const int pr_kt = g ? it.pr_kt[1] : it.pr_kt[0];
     constexpr int NB = kSlices<W>, WS = W / NB;  // columns of a slice
     __shared__ acc_t red[kWaves][64][WS];
-    __shared__ float btile[kWaves][16 * kBTileStride];  // B tiles (FP32 on MFMA only)
+    __shared__ alignas(16) char btile[kWaves][BTile<TS, W>::BYTES];
     const TS* panel = static_cast<const TS*>(I.panel);
     const s_t* S = static_cast<const s_t*>(I.S);
     PanelAcc<TS, W> acc[4 * NB];
@@ -771,7 +688,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_far(const FarItem* __restric
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));  // uniform
     if (wave >= it.nrg) return;
-    __shared__ float btile[kWaves][16 * kBTileStride];  // B tiles (FP32, 16 RHS only)
+    __shared__ alignas(16) char btile[kWaves][BTile<TS, W>::BYTES];
     const int rows = wave == it.nrg - 1 ? it.rows_last : 64;
     const TS* pd = static_cast<const TS*>(I.panel) + it.data_off +
                    static_cast<int64_t>(wave) * 64 * it.ktiles * TK;
