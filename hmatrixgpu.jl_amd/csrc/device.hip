@@ -71,17 +71,19 @@ int64_t leaf_item_work(const PairItem& it) {
 // Size of the k-range pieces that leaf items are cut into, from the leaf bytes of
 // the operator: total / kLeafPieces, at least 1 MiB, so that no item outlasts the
 // launch (swept at N = 262,144).  An operator of at most kSmallLeaf bytes has fewer
-// whole items than the 1,024 workgroups that are resident; it takes total /
-// kSmallPieces, between 128 and 256 KiB.  Measured on the leaf kernel: N = 4,096
-// FP64 with one right-hand side 53 -> 29 us, FP32 with 16 43 -> 18 us; 64 KiB
-// pieces are slower again (start-up of each piece, about 5 us of one workgroup).
-// The line lies where a batch of such operators, which fills the GPU without
-// cutting its members (and must cut them as their own products do, for the same
-// bits), starts to pay for that start-up: 16 members of 2,048 .. 16,384 points take
-// 498 us with 1 MiB pieces, 500 us with this rule, 509 us with twice these limits.
+// whole items than the workgroups that are resident, or too few rounds of them; it takes
+// total / kSmallPieces, between 64 and 384 KiB.  us per product with 1 MiB pieces and with
+// this rule: N = 4,096 FP64 with one right-hand side 78 and 39, FP32 with 16 47 and 29;
+// N = 14,000 FP32 with four 130 and 119; N = 16,384 BF16 with 16 109 and 98; N = 20,011
+// FP32 with three 187 and 182.  Finer pieces pay for their start-up, about 5 us of one
+// workgroup each, and a batch of such operators, which fills the GPU without cutting its
+// members (and must cut them as their own products do, for the same bits), pays for every
+// one: 16 members of 2,048 .. 16,384 points take 461 us with 1 MiB pieces, 473 us with at
+// most 384 KiB, 484 us with at most 256 KiB.  Above the line the larger pieces are as
+// good for one product too (N = 16,384 FP64 with 40: 437 against 450 us).
 constexpr int64_t kLeafPieces = 12288, kSmallPieces = 512;
 constexpr int64_t kMiB = int64_t(1) << 20;
-constexpr int64_t kSmallLeaf = 160 * kMiB;
+constexpr int64_t kSmallLeaf = 800 * kMiB;
 constexpr int kMaxPieces = 64;
 // Target rows up to which an operator without cut items writes Y from the leaf
 // kernel: scattered stores, but one launch less (N = 1,000, one right-hand side:
@@ -96,7 +98,7 @@ int64_t leaf_piece_bytes(int64_t total, int64_t pieces) {
         min_env ? std::max<int64_t>(4096, std::atoll(min_env))
         : total > kSmallLeaf
             ? kMiB
-            : std::min(kMiB / 4, std::max(kMiB / 8, total / kSmallPieces));
+            : std::min(kMiB * 3 / 8, std::max(kMiB / 16, total / kSmallPieces));
     return std::max(total / pieces, min_piece);
 }
 
