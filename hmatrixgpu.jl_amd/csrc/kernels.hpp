@@ -659,10 +659,14 @@ __global__ __launch_bounds__(256) void k_finish(const InstDesc one,
 }
 
 // Far-field work item: up to kWaves consecutive 64-row groups of the stacked V
-// rows of one source cluster over one column chunk.  Wave w owns row group w
-// and walks every k-tile of the chunk; the waves read the same S rows (the
-// cluster's X rows), so the B operand is fetched once per workgroup and shared
-// through the L1 cache.  No cross-wave reduction is needed.
+// rows of one source cluster over one column chunk.  With three or four row groups
+// wave w owns row group w and walks every k-tile of the chunk; the waves read the same S
+// rows (the cluster's X rows), so the B operand is fetched once per workgroup and shared
+// through the L1 cache.  With one or two, four or two waves share a row group's
+// k-tiles and are summed through LDS: one wave alone walked the whole chunk while the
+// others had nothing to do, which set the time of small operators (and of the last
+// item of a cluster).  N = 12,000 on a circle, FP64: far kernel 68 -> 24 us; N = 4,000
+// FP64 with 40 right-hand sides 21 -> 16 us.
 struct FarItem {
     int64_t data_off;  // panel of row group 0; group g at + g*64*ktiles*TK
     int64_t col_off;   // first S row of the chunk
@@ -687,33 +691,55 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_far(const FarItem* __restric
     const InstDesc& I = inst_of<BATCH>(one, insts, it.inst);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));  // uniform
-    if (wave >= it.nrg) return;
+    const int split = it.nrg == 1 ? 4 : it.nrg == 2 ? 2 : 1;  // waves per row group
+    const int g = wave / split;
+    if (g >= it.nrg) return;  // three row groups: no barrier below
+    constexpr int NB = kSlices<W>, WS = W / NB;
     __shared__ alignas(16) char btile[kWaves][BTile<TS, W>::BYTES];
-    const int rows = wave == it.nrg - 1 ? it.rows_last : 64;
+    __shared__ acc_t red[kWaves][64][WS];
+    const int rows = g == it.nrg - 1 ? it.rows_last : 64;
     const TS* pd = static_cast<const TS*>(I.panel) + it.data_off +
-                   static_cast<int64_t>(wave) * 64 * it.ktiles * TK;
-    const int64_t orow = it.out_off + 64 * wave;
+                   static_cast<int64_t>(g) * 64 * it.ktiles * TK;
     s_t* S = static_cast<s_t*>(I.S);
     acc_t* partial = static_cast<acc_t*>(I.partial);
-    constexpr int NB = kSlices<W>;
+    // result of row `row` of the item, column c
+    auto store = [&](int row, int c, acc_t v) {
+        const int64_t o = it.out_off + row;
+        if (it.to_T)
+            S[(I.s0 + I.n + o) * W + c] = from_double<s_t>(static_cast<double>(v));
+        else
+            partial[o * W + c] = v;
+    };
     PanelAcc<TS, W> acc[4 * NB];
 #pragma unroll
     for (int q = 0; q < 4 * NB; q++) acc[q] = PanelAcc<TS, W>{};
     dispatch_nrt(rows, [&](auto nrt) {
         panel_accum<TS, W, false, decltype(nrt)::value, CP, WIDE>(
-            pd, rows, it.ktiles, it.col_off, it.ncols, nullptr, 0, 0, S, I.s_rows, 0, 1, lane,
-            btile[wave], acc);
+            pd, rows, it.ktiles, it.col_off, it.ncols, nullptr, 0, 0, S, I.s_rows, wave % split, split,
+            lane, btile[wave], acc);
     });
+    if (split == 1) {
 #pragma unroll
-    for (int b = 0; b < NB; b++)
-        panel_emit<TS, W>(acc, (rows + 15) >> 4, b, lane, [&](int row, int j, acc_t v) {
-            if (row >= rows) return;
-            const int c = 16 * b + j;
-            if (it.to_T)
-                S[(I.s0 + I.n + orow + row) * W + c] = from_double<s_t>(static_cast<double>(v));
-            else
-                partial[(orow + row) * W + c] = v;
-        });
+        for (int b = 0; b < NB; b++)
+            panel_emit<TS, W>(acc, (rows + 15) >> 4, b, lane, [&](int row, int j, acc_t v) {
+                if (row < rows) store(64 * g + row, WS * b + j, v);
+            });
+        return;
+    }
+    const int total = 64 * (it.nrg - 1) + it.rows_last;
+#pragma unroll
+    for (int b = 0; b < NB; b++) {  // one slice at a time through LDS
+        if (b) __syncthreads();
+        panel_emit<TS, W>(acc, (rows + 15) >> 4, b, lane,
+                          [&](int row, int j, acc_t v) { red[wave][row][j] = v; });
+        __syncthreads();
+        for (int t = threadIdx.x; t < total * WS; t += kWaves * 64) {
+            const int row = t / WS, j = t % WS, w0 = row / 64 * split;
+            acc_t v = red[w0][row % 64][j];
+            for (int w = 1; w < split; w++) v += red[w0 + w][row % 64][j];
+            store(row, WS * b + j, v);
+        }
+    }
 }
 
 // Sum the column-chunk partials of far-field row groups in a fixed order.
