@@ -295,7 +295,7 @@ void device_build(HMatrix& h, int storage) {
     // overrides it.
     const char* ch_env = std::getenv("HMX_FAR_CHUNK");
     const int64_t ch_req = ch_env ? std::atoll(ch_env) : 8192;
-    const int64_t CH = ch_req >= 32 && ch_req % 32 == 0 ? ch_req : 8192;
+    int64_t CH = ch_req >= 32 && ch_req % 32 == 0 ? ch_req : 8192;
 
     // -- far field: group low-rank blocks by source cluster -----------------------
     // Per source cluster the rank rows of its blocks are stacked (T rows, in
@@ -312,6 +312,24 @@ void device_build(HMatrix& h, int storage) {
         std::map<int64_t, std::vector<int64_t>> by_src;
         for (size_t b = 0; b < h.lowrank.size(); b++)
             if (h.lowrank[b].k > 0) by_src[h.lowrank[b].snode].push_back(static_cast<int64_t>(b));
+        // Where the far field is a few long, thin panels (points on a curve: rank 3 or
+        // 4), the longest chain of k-tiles sets the time of its launch: about 0.12 us per
+        // tile of one wave, against far bytes / 6 TB/s for the launch as a whole.  Such an
+        // operator takes 128 k-tiles per chunk (FP64 on a circle: N = 20,000 49 -> 28 us per
+        // product, N = 12,000 33 -> 25 us; operators in a volume never do).
+        if (!ch_env) {
+            double bytes = 0, chain = 0;
+            for (auto& kv : by_src) {
+                const LowRankBlock& f = h.lowrank[kv.second[0]];
+                const int64_t ncols = f.c1 - f.c0 + 1;
+                int64_t Rs = 0;
+                for (int64_t b : kv.second) Rs += h.lowrank[b].k;
+                const int64_t nrg = (Rs + 63) / 64, split = nrg == 1 ? 4 : nrg == 2 ? 2 : 1;
+                bytes += double(Rs) * ncols * elem_size(storage);
+                chain = std::max(chain, double(std::min(ncols, CH)) / (TK * split));
+            }
+            if (chain * 0.12 > 8.0 + 2.0 * bytes / 6e6) CH = 128 * TK;
+        }
         int64_t t = 0;
         for (auto& kv : by_src) {
             const auto& blocks = kv.second;
