@@ -89,6 +89,13 @@ constexpr int kMaxPieces = 64;
 // kernel: scattered stores, but one launch less (N = 1,000, one right-hand side:
 // 17.3 -> 14.5 us per product).
 constexpr int64_t kDirectRows = 8192;
+// Source rows and panel bytes up to which a product with one right-hand side reads X in
+// place, without the gather launch (about 3 us).  A larger operator reads each X row many
+// times, through scattered loads where S has it in tree order.  us per product, gathered
+// and in place: circle N = 1,000 FP64 15.0 and 12.1, N = 4,000 17.8 and 14.8; cube N =
+// 1,200 FP64 17.3 and 14.4, N = 4,096 BF16 (30 MB) 17.8 and 16.0, but N = 2,500 FP64
+// (48 MB) 24.0 and 26.1, N = 12,000 on the circle 24.3 and 25.8.
+constexpr int64_t kXdirRows = 8192, kXdirBytes = 32 * kMiB;
 
 int64_t leaf_piece_bytes(int64_t total, int64_t pieces) {
     // HMX_LEAF_MIN_PIECE sets the smallest piece (bytes), e.g. to split the
@@ -232,7 +239,7 @@ void device_destroy(DeviceOp* op) {
     if (!op) return;
     (void)hipSetDevice(op->device);
     for (void* p : {op->panel, (void*)op->itemsB, (void*)op->colidx, (void*)op->itemsA,
-                    (void*)op->groups, (void*)op->tmap0, (void*)op->rowsrc, (void*)op->inv_smap})
+                    (void*)op->groups, (void*)op->tmap0, (void*)op->rowsrc, (void*)op->inv_smap, (void*)op->smap0, (void*)op->colx})
         if (p) (void)hipFree(p);
     for (auto& kv : op->scratch)
         for (auto& w : kv.second.w)
@@ -254,7 +261,8 @@ int64_t device_index_bytes(const DeviceOp* op) {
     return op->ncol * 4 + op->nA * static_cast<int64_t>(sizeof(FarItem)) +
            op->nB * static_cast<int64_t>(sizeof(PairItem)) +
            op->nG * static_cast<int64_t>(sizeof(ReduceGroup)) +
-           op->m * static_cast<int64_t>(4 + sizeof(RowSrc)) + op->n * 4;
+           op->m * static_cast<int64_t>(4 + sizeof(RowSrc)) + op->n * 4 +
+           (op->colx ? (op->ncol + op->n) * 4 : 0);
 }
 
 // Build the device operator for one storage precision.
@@ -586,6 +594,14 @@ void device_build(HMatrix& h, int storage) {
     for (int64_t i = 0; i < h.n; i++) inv[h.smap[i] - 1] = static_cast<int32_t>(i);
     op->tmap0 = upload(tmap0);
     op->inv_smap = upload(inv);
+    if (h.n <= kXdirRows && data_off * static_cast<int64_t>(elem_size(storage)) <= kXdirBytes && s0 == 0) {
+        std::vector<int32_t> smap0(h.n), colx(colidx);
+        for (int64_t i = 0; i < h.n; i++) smap0[i] = static_cast<int32_t>(h.smap[i] - 1);
+        for (int32_t& c : colx)
+            if (c < h.n) c = smap0[c];
+        op->smap0 = upload(smap0);
+        op->colx = upload(colx);
+    }
     // The FP64 staging arrays are allocated before the panel and freed after
     // generation.  Measured on the MI355X, the product's speed depends on where
     // the panel allocation lands relative to the other large buffers of the
@@ -770,6 +786,16 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     return s;
 }
 
+// Whether a product reads X in place: one right-hand side of the accumulation type, a
+// small operator, and a Y that does not overlap X (the leaf kernel writes Y while
+// others still read X).
+template <typename TS, int W, typename TIO>
+bool reads_x_in_place(const DeviceOp& op, const void* X, const void* Y) {
+    if (W != 1 || !op.colx || !std::is_same<TIO, typename Store<TS>::acc>::value) return false;
+    const uintptr_t x = reinterpret_cast<uintptr_t>(X), y = reinterpret_cast<uintptr_t>(Y);
+    return x + op.n * sizeof(TIO) <= y || y + op.m * sizeof(TIO) <= x;
+}
+
 template <typename TS, int W, typename TIO>
 void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs, hipStream_t st) {
     ScratchW& sc = get_scratch(op, st, W);
@@ -785,6 +811,8 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
     one.m = op.m;
     one.tmap0 = op.tmap0;
     one.inv_smap = op.inv_smap;
+    one.smap0 = op.smap0;
+    one.colx = op.colx;
     one.X = X;
     one.Y = Y;
     one.ldx = ldx;
@@ -804,6 +832,7 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
     A.gather_n = op.n;
     A.gather_insts = 1;
     A.wide = wide_staging(lay);
+    A.xdir = !A.wide && reads_x_in_place<TS, W, TIO>(op, X, Y);
     A.out_m = op.direct ? 0 : op.m;
     for (int rhs0 = 0; rhs0 < nrhs; rhs0 += W) {
         one.rhs0 = rhs0;
@@ -940,6 +969,8 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
     one.m = op.m;
     one.tmap0 = op.tmap0;
     one.inv_smap = op.inv_smap;
+    one.smap0 = op.smap0;
+    one.colx = op.colx;
     one.X = X;
     one.Y = Y;
     one.ldx = ldx;
@@ -960,6 +991,7 @@ void run_noalloc(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy,
     A.gather_n = op.n;
     A.gather_insts = 1;
     A.wide = wide_staging(lay);
+    A.xdir = !A.wide && reads_x_in_place<TS, W, TIO>(op, X, Y);
     A.out_m = op.direct ? 0 : op.m;
     for (int rhs0 = 0; rhs0 < nrhs; rhs0 += W) {
         one.rhs0 = rhs0;

@@ -40,6 +40,8 @@ struct DeviceOp {
     bool direct = false;        // the leaf kernel writes Y (no item is cut, few rows)
     int32_t* tmap0 = nullptr;
     int32_t* inv_smap = nullptr;
+    int32_t* smap0 = nullptr;   // small operators only (xdir): permuted source -> original row
+    int32_t* colx = nullptr;    // and the leaf columns with X by original row
     // host copies of the work lists (the batched operator re-packs them)
     std::vector<PairItem> hItemsB;
     std::vector<FarItem> hItemsA;
@@ -99,6 +101,7 @@ struct StageArrays {
     int gather_insts = 1;   // instances (grid.y of the gather and the unpermute)
     int64_t out_m = 0;      // largest target size over the instances that need k_finish
     bool wide = false;      // an instance's S has 4 GiB or more: 64-bit S loads
+    bool xdir = false;      // X is read in place (one right-hand side): no gather
 };
 // S of 4 GiB or more: beyond the reach of 32-bit buffer offsets
 inline bool wide_staging(const StagingLayout& L) { return L.bytes >= (int64_t(1) << 32); }
@@ -130,13 +133,22 @@ struct StageTimer {
 template <typename TS, int W, typename TIO, bool BATCH>
 void launch_stages(const StageArrays& A, const InstDesc& one, const InstDesc* insts,
                    hipStream_t st, DeviceOp* prof) {
-    {
+    if constexpr (W == 1 && !BATCH && std::is_same<TIO, typename Store<TS>::acc>::value) {
+        if (A.xdir) {
+            if (A.nA) {
+                StageTimer t(prof, st, 1);
+                hipLaunchKernelGGL((k_far<TS, 1, kPanelPolicy, false, false, true>), dim3(A.nA),
+                                   dim3(kWaves * 64), 0, st, A.itemsA, one, insts);
+            }
+        }
+    }
+    if (!A.xdir) {
         StageTimer t(prof, st, 0);
         hipLaunchKernelGGL((k_gather<TS, W, TIO, BATCH>),
                            dim3(static_cast<unsigned>((A.gather_n + 255) / 256), A.gather_insts),
                            dim3(256), 0, st, one, insts);
     }
-    if (A.nA) {
+    if (A.nA && !A.xdir) {
         StageTimer t(prof, st, 1);
         if (A.wide)
             hipLaunchKernelGGL((k_far<TS, W, kPanelPolicy, BATCH, true>), dim3(A.nA),
@@ -150,7 +162,14 @@ void launch_stages(const StageArrays& A, const InstDesc& one, const InstDesc* in
         hipLaunchKernelGGL((k_reduce<TS, W, BATCH>), dim3(A.nG), dim3(256), 0, st, A.groups, one,
                            insts);
     }
-    if (A.nB) {
+    if constexpr (W == 1 && !BATCH && std::is_same<TIO, typename Store<TS>::acc>::value) {
+        if (A.nB && A.xdir) {
+            StageTimer t(prof, st, 3);
+            hipLaunchKernelGGL((k_leaf<TS, 1, kPanelPolicy, false, false, true>), dim3(A.nB),
+                               dim3(kWaves * 64), 0, st, A.itemsB, one, insts);
+        }
+    }
+    if (A.nB && !A.xdir) {
         StageTimer t(prof, st, 3);
         if (A.wide)
             hipLaunchKernelGGL((k_leaf<TS, W, kPanelPolicy, BATCH, true>), dim3(A.nB),

@@ -94,6 +94,8 @@ struct InstDesc {
     int64_t m;               // target rows
     const int32_t* tmap0;    // permuted target row -> 0-based original row
     const int32_t* inv_smap; // 0-based original source row -> permuted row
+    const int32_t* smap0;    // permuted source row -> 0-based original row
+    const int32_t* colx;     // colidx with the X columns by original row (XDIR), or null
     const void* X;
     void* Y;
     int64_t ldx, ldy;
@@ -246,6 +248,10 @@ struct alignas(sizeof(T) * W >= 16 ? 16 : sizeof(T) * W) SRowOut {
 // colidx + pr_off for the rest) or as the contiguous rows col_off + k masked
 // beyond ncols.  The
 // accumulated results are handed to emit(row, col, value), row < 64, col < W.
+// XDIR (one right-hand side, X of the accumulation type, a small operator): X is read
+// from the caller's vector instead of S.  A column index below n then is a row of X
+// (LEAF: from the index array; far field: col_off addresses smap0), any other one a row
+// of S; each is one load that the other's range check turns into zeros.
 // W = 16 runs on MFMA (16 right-hand sides as the N dimension); W = 1 and 4 run
 // on the VALU, lane (row li, k-chunk lg).  Loads are issued one k-tile ahead (A
 // and B) and two ahead (column indices).  CP is the cache policy of the
@@ -259,13 +265,14 @@ using PanelAcc = typename std::conditional<
                               f32x4>::type,
     SRow<typename Store<TS>::acc, W>>::type;
 
-template <typename TS, int W, bool LEAF, int NRT, int CP, bool WIDE>
+template <typename TS, int W, bool LEAF, int NRT, int CP, bool WIDE, bool XDIR = false>
 __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktiles, int64_t col_off,
                                             int ncols, const int32_t* colidx, int sh_kt,
                                             int64_t pr_off,
                                             const typename SType<TS, W>::type* S, uint32_t s_rows,
                                             int kt0, int kstep, int lane, char* btile,
-                                            PanelAcc<TS, W>* acc) {
+                                            PanelAcc<TS, W>* acc, const void* X = nullptr,
+                                            int64_t n = 0) {
     using acc_t = typename Store<TS>::acc;
     using s_t = typename SType<TS, W>::type;
     constexpr int TK = Store<TS>::TK, EPL = Store<TS>::EPL;
@@ -276,9 +283,13 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
     const __amdgpu_buffer_rsrc_t Sr = make_rsrc(S, WIDE ? 0u : s_rows * ROWB);
     // Column indices of both segments, addressed by the k-tile of the whole
     // panel: the private ones from a base moved back by the shared tiles.
-    const int32_t* const csh = colidx + (LEAF ? col_off : 0);
+    const int32_t* const csh = colidx + (LEAF || XDIR ? col_off : 0);
     const int32_t* const cpr = colidx + (LEAF ? pr_off - static_cast<int64_t>(sh_kt) * TK : 0);
-    const __amdgpu_buffer_rsrc_t Csh = make_rsrc(csh, ktiles * TK * 4), Cpr = make_rsrc(cpr, ktiles * TK * 4);
+    const __amdgpu_buffer_rsrc_t Csh = make_rsrc(csh, (LEAF ? ktiles * TK : ncols) * 4),
+                                 Cpr = LEAF ? make_rsrc(cpr, ktiles * TK * 4) : Csh;
+    const __amdgpu_buffer_rsrc_t Xr = make_rsrc(X, static_cast<uint32_t>(n) * ROWB);
+    constexpr bool INDEXED = LEAF || XDIR;  // columns come through an index array
+    static_assert(!XDIR || (W == 1 && !WIDE), "XDIR: one right-hand side, S below 4 GiB");
     uint32_t aoff[NRT];
     bool aval[NRT];
 #pragma unroll
@@ -328,6 +339,24 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
             const int k = kt * TK + brow;
             ok = ok && k < ncols;
             row = ok ? static_cast<uint32_t>(col_off + k) : s_rows - 1;
+        }
+        if constexpr (XDIR) {
+            const uint32_t r = static_cast<uint32_t>(LEAF ? row : ix);
+            const uint32_t xo = ok && r < static_cast<uint32_t>(n) ? r * ROWB : kOOB;
+            const uint32_t so = LEAF && ok && r >= static_cast<uint32_t>(n) ? r * ROWB : kOOB;
+            part_t v;
+            if constexpr (BT::LB == 8)
+                v = __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b64(Xr, xo, 0, 0));
+            else
+                v = __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b32(Xr, xo, 0, 0));
+            if constexpr (LEAF) {  // the one that is out of range reads zeros
+                if constexpr (BT::LB == 8)
+                    v |= __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b64(Sr, so, 0, 0));
+                else
+                    v |= __builtin_bit_cast(part_t, __builtin_amdgcn_raw_buffer_load_b32(Sr, so, 0, 0));
+            }
+            st.b[0] = v;
+            return st;
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
@@ -460,7 +489,7 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
 #pragma unroll
     for (int d = 0; d < D; d++) {
         ix[d] = 0;
-        if constexpr (LEAF) ix[d] = load_ix(kt + d * kstep);
+        if constexpr (INDEXED) ix[d] = load_ix(kt + d * kstep);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -468,14 +497,14 @@ __device__ __forceinline__ void panel_accum(const TS* pdata, int rows, int ktile
         st[d] = load_stage(kt + d * kstep, ix[d]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (LEAF) ix[0] = load_ix(kt + D * kstep);
+    if constexpr (INDEXED) ix[0] = load_ix(kt + D * kstep);
     __builtin_amdgcn_sched_barrier(0);
     int i = 0;
     for (; i + D - 1 < mine; i += D) {
 #pragma unroll
         for (int j = 0; j < D; j++) {
             st[(j + D - 1) % D] = load_stage(kt + (j + D - 1) * kstep, ix[(j + D - 1) % D]);
-            if constexpr (LEAF) ix[(j + 1) % D] = load_ix(kt + (j + D + 1) * kstep);
+            if constexpr (INDEXED) ix[(j + 1) % D] = load_ix(kt + (j + D + 1) * kstep);
             compute(st[j]);
         }
         kt += D * kstep;
@@ -544,7 +573,7 @@ __device__ __forceinline__ const InstDesc& inst_of(const InstDesc& one, const In
 // single row group is split over all four waves.  Partial sums are reduced
 // through LDS and written as whole leaf-result rows, which k_finish sums and
 // scatters; the items of a small operator, none of them cut, write Y directly.
-template <typename TS, int W, int CP, bool BATCH, bool WIDE>
+template <typename TS, int W, int CP, bool BATCH, bool WIDE, bool XDIR = false>
 __global__ __launch_bounds__(kWaves * 64, 2) void k_leaf(const PairItem* __restrict__ items,
                                                       const InstDesc one,
                                                       const InstDesc* __restrict__ insts) {
@@ -575,9 +604,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_leaf(const PairItem* __restr
     for (int q = 0; q < 4 * NB; q++) acc[q] = PanelAcc<TS, W>{};
     dispatch_nrt(rows, [&](auto nrt) {
         constexpr int NRT = decltype(nrt)::value;
-        panel_accum<TS, W, true, NRT, CP, WIDE>(panel + data, rows, it.sh_kt + pr_kt, it.sh_col, 0,
-                                                I.colidx, it.sh_kt, pr_col, S, I.s_rows, kt0, kstep,
-                                                lane, btile[wave], acc);
+        panel_accum<TS, W, true, NRT, CP, WIDE, XDIR>(panel + data, rows, it.sh_kt + pr_kt, it.sh_col,
+                                                      0, XDIR ? I.colx : I.colidx, it.sh_kt, pr_col, S,
+                                                      I.s_rows, kt0, kstep, lane, btile[wave], acc,
+                                                      I.X, I.n);
     });
     acc_t* lrows = static_cast<acc_t*>(I.lrows);
     const int r0 = it.rows[0], total = r0 + it.rows[1];
@@ -680,7 +710,7 @@ struct FarItem {
     int32_t pad;
 };
 
-template <typename TS, int W, int CP, bool BATCH, bool WIDE>
+template <typename TS, int W, int CP, bool BATCH, bool WIDE, bool XDIR = false>
 __global__ __launch_bounds__(kWaves * 64, 2) void k_far(const FarItem* __restrict__ items,
                                                      const InstDesc one,
                                                      const InstDesc* __restrict__ insts) {
@@ -714,9 +744,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_far(const FarItem* __restric
 #pragma unroll
     for (int q = 0; q < 4 * NB; q++) acc[q] = PanelAcc<TS, W>{};
     dispatch_nrt(rows, [&](auto nrt) {
-        panel_accum<TS, W, false, decltype(nrt)::value, CP, WIDE>(
-            pd, rows, it.ktiles, it.col_off, it.ncols, nullptr, 0, 0, S, I.s_rows, wave % split, split,
-            lane, btile[wave], acc);
+        panel_accum<TS, W, false, decltype(nrt)::value, CP, WIDE, XDIR>(
+            pd, rows, it.ktiles, it.col_off, it.ncols, XDIR ? I.smap0 : nullptr, 0, 0, S, I.s_rows,
+            wave % split, split, lane, btile[wave], acc, I.X, I.n);
     });
     if (split == 1) {
 #pragma unroll
