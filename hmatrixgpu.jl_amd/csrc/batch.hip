@@ -86,11 +86,8 @@ ScratchW& batch_scratch(Batch& b, size_t i, int W) {
     ScratchW& s = v[i];
     if (!s.S) {
         const DeviceOp& op = *b.ops[i];
-        const size_t sb = static_cast<size_t>(staging(op, W).zero_end);
-        HIPCHECK(hipMalloc(&s.S, sb));
+        alloc_scratch(op, W, s);
         zero_staging_tail(s.S, staging(op, W), nullptr);
-        HIPCHECK(hipMalloc(&s.P, std::max<int64_t>(op.npartial, 1) * W * p_elem(op.storage)));
-        HIPCHECK(hipMalloc(&s.LP, std::max<int64_t>(op.nlrows, 1) * W * p_elem(op.storage)));
     }
     return s;
 }
@@ -283,8 +280,7 @@ Batch::~Batch() {
         if (p) (void)hipHostFree(p);
     for (auto& v : scratch)
         for (auto& s : v)
-            for (void* p : {s.S, s.P, s.LP})
-                if (p) (void)hipFree(p);
+            if (s.S) (void)hipFree(s.S);
     if (cap_stream) (void)hipStreamDestroy(cap_stream);
 }
 

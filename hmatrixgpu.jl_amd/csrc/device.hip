@@ -243,8 +243,7 @@ void device_destroy(DeviceOp* op) {
         if (p) (void)hipFree(p);
     for (auto& kv : op->scratch)
         for (auto& w : kv.second.w)
-            for (void* p : {w.S, w.P, w.LP})
-                if (p) (void)hipFree(p);
+            if (w.S) (void)hipFree(w.S);
     for (auto& e : op->ev)
         for (auto& pr : e) {
             (void)hipEventDestroy(pr.first);
@@ -735,15 +734,13 @@ size_t scratch_stream_limit() {
 
 void free_scratch(Scratch& sc) {
     for (auto& w : sc.w)
-        for (void* p : {w.S, w.P, w.LP})
-            if (p) HIPCHECK(hipFree(p));
+        if (w.S) HIPCHECK(hipFree(w.S));
     sc = Scratch{};
 }
 
 // Per-stream scratch of one pass width, allocated on the stream's first call:
-// the size is checked before anything is allocated, and the arrays are kept only when all of them were allocated.
+// in one allocation.
 ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
-    const size_t sb = static_cast<size_t>(staging(op, W).zero_end);
     std::lock_guard<std::mutex> g(op.mu);
     auto it = op.scratch.find(static_cast<void*>(stream));
     if (it == op.scratch.end()) {
@@ -762,26 +759,21 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     ScratchW& s = it->second.w[w_slot(W)];
     if (!s.S) {
         ScratchW n;
-        const size_t pb = std::max<int64_t>(op.npartial, 1) * W * p_elem(op.storage);
-        const size_t lb = std::max<int64_t>(op.nlrows, 1) * W * p_elem(op.storage);
-        try {
-            HIPCHECK(hipMalloc(&n.S, sb));
-            HIPCHECK(hipMalloc(&n.P, pb));
-            HIPCHECK(hipMalloc(&n.LP, lb));
-        } catch (...) {
-            for (void* p : {n.S, n.P, n.LP})
-                if (p) (void)hipFree(p);
-            throw;
-        }
+        const size_t bytes = alloc_scratch(op, W, n);
         // On the product's own stream: a clear on the null stream is not ordered
         // before the work of a stream created without that dependence, and would
         // overwrite rows that the first product has already written.
-        zero_staging_tail(n.S, staging(op, W), stream);
+        try {
+            zero_staging_tail(n.S, staging(op, W), stream);
+        } catch (...) {
+            (void)hipFree(n.S);
+            throw;
+        }
         s = n;
-        it->second.bytes += sb + pb + lb;
+        it->second.bytes += bytes;
         if (std::getenv("HMX_VERBOSE"))
-            std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p (%zu bytes), partials %p\n",
-                         op.storage, W, s.S, sb, s.P);
+            std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes)\n",
+                         op.storage, W, s.S, s.P, bytes);
     }
     return s;
 }
@@ -1107,8 +1099,7 @@ int64_t device_release_scratch(HMatrix& h, void* stream, bool all_streams) {
             // the stream's products may still be running
             HIPCHECK(hipStreamSynchronize(static_cast<hipStream_t>(it->first)));
             for (auto& w : it->second.w)
-                for (void* p : {w.S, w.P, w.LP})
-                    if (p) freed++;
+                if (w.S) freed++;
             free_scratch(it->second);
             it = d->scratch.erase(it);
         }

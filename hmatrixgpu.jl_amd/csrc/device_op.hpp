@@ -6,6 +6,7 @@
 
 namespace hmx {
 
+// Scratch of one pass width: three arrays in one allocation, which S is the start of.
 struct ScratchW {
     void* S = nullptr;  // (s0 + n + R + 1 + TK) x W source rows (staging_layout)
     void* P = nullptr;   // far-field partial rows x W
@@ -88,6 +89,19 @@ struct DeviceGuard {
     }
     ~DeviceGuard() { (void)hipSetDevice(prev); }
 };
+
+// Allocate the scratch of one pass width; returns its bytes.
+inline size_t alloc_scratch(const DeviceOp& op, int W, ScratchW& s) {
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t pe = p_elem(op.storage);
+    const size_t sb = up(static_cast<size_t>(staging(op, W).zero_end));
+    const size_t pb = up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe);
+    const size_t lb = up(static_cast<size_t>(std::max<int64_t>(op.nlrows, 1)) * W * pe);
+    HIPCHECK(hipMalloc(&s.S, sb + pb + lb));
+    s.P = static_cast<char*>(s.S) + sb;
+    s.LP = static_cast<char*>(s.P) + pb;
+    return sb + pb + lb;
+}
 
 // Work lists of one launch (one H-matrix, or a batch of them).
 struct StageArrays {

@@ -228,7 +228,7 @@ void device_matvec_noalloc(HMatrix& h, int storage, const void* X, int64_t ldx, 
 void device_matvec_host(HMatrix& h, const double* x, int64_t ldx, double* y, int64_t ldy,
                         int nrhs);
 // Free the per-stream scratch of `stream` (or of every stream) of every storage
-// precision after synchronising those streams; returns the arrays freed.
+// precision after synchronising those streams; returns the allocations freed.
 int64_t device_release_scratch(HMatrix& h, void* stream, bool all_streams);
 // bytes of product scratch held and (operator, stream) entries holding it
 void device_scratch_usage(const HMatrix& h, int64_t* bytes, int64_t* entries);
