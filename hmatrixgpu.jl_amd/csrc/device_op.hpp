@@ -112,7 +112,7 @@ struct StageArrays {
     const PairItem* itemsB = nullptr;
     int64_t nB = 0;
     int64_t gather_n = 0;   // largest source size over the instances
-    int gather_insts = 1;   // instances (grid.y of the gather and the unpermute)
+    int gather_insts = 1;   // instances (grid.y of the gather and the finish)
     int64_t out_m = 0;      // largest target size over the instances that need k_finish
     bool wide = false;      // an instance's S has 4 GiB or more: 64-bit S loads
     bool xdir = false;      // X is read in place (one right-hand side): no gather

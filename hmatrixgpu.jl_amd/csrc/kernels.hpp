@@ -252,12 +252,11 @@ struct alignas(sizeof(T) * W >= 16 ? 16 : sizeof(T) * W) SRowOut {
 // from the caller's vector instead of S.  A column index below n then is a row of X
 // (LEAF: from the index array; far field: col_off addresses smap0), any other one a row
 // of S; each is one load that the other's range check turns into zeros.
-// W = 16 runs on MFMA (16 right-hand sides as the N dimension); W = 1 and 4 run
-// on the VALU, lane (row li, k-chunk lg).  Loads are issued one k-tile ahead (A
-// and B) and two ahead (column indices).  CP is the cache policy of the
-// streamed A loads.
-// Accumulator of one wave over NRT 16-row tiles: MFMA C/D registers (W = 16)
-// or per-lane partial sums (W = 1, 4).
+// W = 16, 32 and 48 run on MFMA (16 right-hand sides as the N dimension of each of NB
+// slices); W = 1 and 4 run on the VALU, lane (row li, k-chunk lg).  CP is the cache
+// policy of the streamed A loads.
+// Accumulator of one wave for one 16-row tile and slice: MFMA C/D registers, or
+// per-lane partial sums (W = 1, 4); acc[rt * NB + slice].
 template <typename TS, int W>
 using PanelAcc = typename std::conditional<
     kMfma<W>,
