@@ -758,18 +758,7 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     it->second.last_use = ++op.use_clock;
     ScratchW& s = it->second.w[w_slot(W)];
     if (!s.S) {
-        ScratchW n;
-        const size_t bytes = alloc_scratch(op, W, n);
-        // On the product's own stream: a clear on the null stream is not ordered
-        // before the work of a stream created without that dependence, and would
-        // overwrite rows that the first product has already written.
-        try {
-            zero_staging_tail(n.S, staging(op, W), stream);
-        } catch (...) {
-            (void)hipFree(n.S);
-            throw;
-        }
-        s = n;
+        const size_t bytes = alloc_scratch(op, W, stream, s);
         it->second.bytes += bytes;
         if (std::getenv("HMX_VERBOSE"))
             std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes)\n",

@@ -90,16 +90,51 @@ struct DeviceGuard {
     ~DeviceGuard() { (void)hipSetDevice(prev); }
 };
 
-// Allocate the scratch of one pass width; returns its bytes.
-inline size_t alloc_scratch(const DeviceOp& op, int W, ScratchW& s) {
+// Clear the zero and padding rows of new scratch, so that whatever runs next on `st`
+// reads zeros.  On that stream itself: a clear on the null stream is not ordered before
+// the work of a stream created without that dependence, and would overwrite rows that the
+// first product has already written.  While `st` is being captured (a relaxed capture may
+// allocate) the launch would only be recorded, and a product that runs before the graph
+// does would read uncleared rows; the clear then runs at once on a stream of its own.
+inline void clear_new_staging(void* S, const StagingLayout& lay, hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+        zero_staging_tail(S, lay, st);
+        return;
+    }
+    (void)hipGetLastError();
+    hipStream_t own = nullptr;
+    HIPCHECK(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
+    try {
+        zero_staging_tail(S, lay, own);
+        HIPCHECK(hipStreamSynchronize(own));
+    } catch (...) {
+        (void)hipStreamDestroy(own);
+        throw;
+    }
+    HIPCHECK(hipStreamDestroy(own));
+}
+
+// Allocate the scratch of one pass width, with its zero rows cleared before anything
+// else on `st`; returns its bytes.  `s` is set only when both have succeeded.
+inline size_t alloc_scratch(const DeviceOp& op, int W, hipStream_t st, ScratchW& s) {
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t pe = p_elem(op.storage);
-    const size_t sb = up(static_cast<size_t>(staging(op, W).zero_end));
+    const StagingLayout lay = staging(op, W);
+    const size_t sb = up(static_cast<size_t>(lay.zero_end));
     const size_t pb = up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe);
     const size_t lb = up(static_cast<size_t>(std::max<int64_t>(op.nlrows, 1)) * W * pe);
-    HIPCHECK(hipMalloc(&s.S, sb + pb + lb));
-    s.P = static_cast<char*>(s.S) + sb;
-    s.LP = static_cast<char*>(s.P) + pb;
+    ScratchW n;
+    HIPCHECK(hipMalloc(&n.S, sb + pb + lb));
+    try {
+        clear_new_staging(n.S, lay, st);
+    } catch (...) {
+        (void)hipFree(n.S);
+        throw;
+    }
+    n.P = static_cast<char*>(n.S) + sb;
+    n.LP = static_cast<char*>(n.P) + pb;
+    s = n;
     return sb + pb + lb;
 }
 
