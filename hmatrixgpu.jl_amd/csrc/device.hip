@@ -738,9 +738,24 @@ void free_scratch(Scratch& sc) {
     sc = Scratch{};
 }
 
+// The scratch of `width` columns in a stream's slots: its own, or (MFMA passes) part of a
+// wider one, whose three arrays are large enough.  The zero rows of every width start
+// at the same address, so they are cleared once and no pass writes them: the narrower S
+// ends with them and begins further back.  A stream that has run a wide product can
+// therefore run, and record into a graph, any narrower one without an allocation.
+ScratchW held_scratch(const DeviceOp& op, const Scratch& sc, int W) {
+    for (int w = W; w <= kMaxWidth && (w == W || W >= 16); w += 16) {
+        ScratchW s = sc.w[w_slot(w)];
+        if (!s.S) continue;
+        s.S = static_cast<char*>(s.S) + staging(op, w).zero_begin - staging(op, W).zero_begin;
+        return s;
+    }
+    return ScratchW{};
+}
+
 // Per-stream scratch of one pass width, allocated on the stream's first call:
 // in one allocation.
-ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
+ScratchW get_scratch(DeviceOp& op, hipStream_t stream, int W) {
     std::lock_guard<std::mutex> g(op.mu);
     auto it = op.scratch.find(static_cast<void*>(stream));
     if (it == op.scratch.end()) {
@@ -756,13 +771,13 @@ ScratchW& get_scratch(DeviceOp& op, hipStream_t stream, int W) {
         it = op.scratch.emplace(static_cast<void*>(stream), Scratch{}).first;
     }
     it->second.last_use = ++op.use_clock;
-    ScratchW& s = it->second.w[w_slot(W)];
+    ScratchW s = held_scratch(op, it->second, W);
     if (!s.S) {
-        const size_t bytes = alloc_scratch(op, W, stream, s);
-        it->second.bytes += bytes;
+        it->second.bytes += alloc_scratch(op, W, stream, s);
+        it->second.w[w_slot(W)] = s;
         if (std::getenv("HMX_VERBOSE"))
-            std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes)\n",
-                         op.storage, W, s.S, s.P, bytes);
+            std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes held)\n",
+                         op.storage, W, s.S, s.P, it->second.bytes);
     }
     return s;
 }
@@ -779,7 +794,7 @@ bool reads_x_in_place(const DeviceOp& op, const void* X, const void* Y) {
 
 template <typename TS, int W, typename TIO>
 void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs, hipStream_t st) {
-    ScratchW& sc = get_scratch(op, st, W);
+    const ScratchW sc = get_scratch(op, st, W);
     InstDesc one{};
     one.panel = op.panel;
     one.colidx = op.colidx;
@@ -836,12 +851,12 @@ int pass_width(int nrhs) {
 
 // Whether a wide pass (32 or 48 columns) can have its scratch: it holds up to three
 // times that of 16 columns.  A stream that is being captured gets no new scratch, and
-// without the memory the product runs in 16-column passes (the same bits).
+// without the memory the product runs in narrower passes (the same bits).
 bool wide_scratch(DeviceOp& op, hipStream_t st, int W) {
     {
         std::lock_guard<std::mutex> g(op.mu);
         auto it = op.scratch.find(static_cast<void*>(st));
-        if (it != op.scratch.end() && it->second.w[w_slot(W)].S) return true;
+        if (it != op.scratch.end() && held_scratch(op, it->second, W).S) return true;
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
@@ -859,14 +874,15 @@ bool wide_scratch(DeviceOp& op, hipStream_t st, int W) {
 
 template <typename TS, typename TIO>
 void run_w(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrhs, hipStream_t st) {
-    const int W = pass_width(nrhs);
+    int W = pass_width(nrhs);
+    while (W > 16 && !wide_scratch(op, st, W)) W -= 16;
     if (W == 1)
         run<TS, 1, TIO>(op, X, ldx, Y, ldy, nrhs, st);
     else if (W == 4)
         run<TS, 4, TIO>(op, X, ldx, Y, ldy, nrhs, st);
-    else if (W == 48 && wide_scratch(op, st, 48))
+    else if (W == 48)
         run<TS, 48, TIO>(op, X, ldx, Y, ldy, nrhs, st);
-    else if (W == 32 && wide_scratch(op, st, 32))
+    else if (W == 32)
         run<TS, 32, TIO>(op, X, ldx, Y, ldy, nrhs, st);
     else
         run<TS, 16, TIO>(op, X, ldx, Y, ldy, nrhs, st);

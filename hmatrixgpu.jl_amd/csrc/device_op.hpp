@@ -19,6 +19,7 @@ struct Scratch {
     size_t bytes = 0;       // bytes held by the arrays of every width
 };
 
+constexpr int kMaxWidth = 48;  // widest pass
 inline int w_slot(int W) { return W == 1 ? 0 : W == 4 ? 1 : 1 + W / 16; }
 
 struct DeviceOp {
