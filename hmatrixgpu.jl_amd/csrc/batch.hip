@@ -84,7 +84,7 @@ ScratchW& batch_scratch(Batch& b, size_t i, int W) {
     auto& v = b.scratch[w_slot(W)];
     if (v.empty()) v.resize(b.ops.size());
     ScratchW& s = v[i];
-    if (!s.S) alloc_scratch(*b.ops[i], W, nullptr, s);
+    if (!s.S) HIPCHECK(alloc_scratch(*b.ops[i], W, nullptr, s));
     return s;
 }
 

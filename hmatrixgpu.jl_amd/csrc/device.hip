@@ -753,10 +753,8 @@ ScratchW held_scratch(const DeviceOp& op, const Scratch& sc, int W) {
     return ScratchW{};
 }
 
-// Per-stream scratch of one pass width, allocated on the stream's first call:
-// in one allocation.
-ScratchW get_scratch(DeviceOp& op, hipStream_t stream, int W) {
-    std::lock_guard<std::mutex> g(op.mu);
+// The scratch entry of a stream (op.mu is held), made on its first call.
+Scratch& stream_scratch(DeviceOp& op, hipStream_t stream) {
     auto it = op.scratch.find(static_cast<void*>(stream));
     if (it == op.scratch.end()) {
         const size_t limit = scratch_stream_limit();
@@ -771,13 +769,27 @@ ScratchW get_scratch(DeviceOp& op, hipStream_t stream, int W) {
         it = op.scratch.emplace(static_cast<void*>(stream), Scratch{}).first;
     }
     it->second.last_use = ++op.use_clock;
-    ScratchW s = held_scratch(op, it->second, W);
+    return it->second;
+}
+
+void keep_scratch(const DeviceOp& op, Scratch& sc, int W, const ScratchW& s) {
+    const size_t bytes = scratch_sizes(op, W).total();
+    sc.w[w_slot(W)] = s;
+    sc.bytes += bytes;
+    if (std::getenv("HMX_VERBOSE"))
+        std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes)\n",
+                     op.storage, W, s.S, s.P, bytes);
+}
+
+// Per-stream scratch of one pass width, allocated on the stream's first call:
+// in one allocation.
+ScratchW get_scratch(DeviceOp& op, hipStream_t stream, int W) {
+    std::lock_guard<std::mutex> g(op.mu);
+    Scratch& sc = stream_scratch(op, stream);
+    ScratchW s = held_scratch(op, sc, W);
     if (!s.S) {
-        it->second.bytes += alloc_scratch(op, W, stream, s);
-        it->second.w[w_slot(W)] = s;
-        if (std::getenv("HMX_VERBOSE"))
-            std::fprintf(stderr, "[hmx] storage %d W %d source/T rows %p, partials %p (%zu bytes held)\n",
-                         op.storage, W, s.S, s.P, it->second.bytes);
+        HIPCHECK(alloc_scratch(op, W, stream, s));
+        keep_scratch(op, sc, W, s);
     }
     return s;
 }
@@ -849,27 +861,48 @@ int pass_width(int nrhs) {
     return 16 * ((nrhs + 16 * passes - 1) / (16 * passes));
 }
 
-// Whether a wide pass (32 or 48 columns) can have its scratch: it holds up to three
-// times that of 16 columns.  A stream that is being captured gets no new scratch, and
-// without the memory the product runs in narrower passes (the same bits).
+// Bytes that the scratch of a wide pass may take: half of the device memory that is
+// free, so that it does not starve the caller's own allocations, or
+// HMX_WIDE_SCRATCH_LIMIT where that is less.
+size_t wide_scratch_limit() {
+    size_t free_b = 0, total_b = 0;
+    HIPCHECK(hipMemGetInfo(&free_b, &total_b));
+    size_t limit = free_b / 2;
+    if (const char* e = std::getenv("HMX_WIDE_SCRATCH_LIMIT")) {
+        const long long v = std::atoll(e);
+        if (v >= 0) limit = std::min(limit, static_cast<size_t>(v));
+    }
+    return limit;
+}
+
+// Whether a wide pass (32 or 48 columns) can have its scratch, two or three times that
+// of 16 columns.  A stream that is being captured gets no new scratch, and where the
+// allocation fails or passes the limit above the product runs in narrower passes (the
+// same bits).  A lack of memory is remembered until the stream's scratch is released,
+// so that not every product tries again.
 bool wide_scratch(DeviceOp& op, hipStream_t st, int W) {
-    {
-        std::lock_guard<std::mutex> g(op.mu);
-        auto it = op.scratch.find(static_cast<void*>(st));
-        if (it != op.scratch.end() && held_scratch(op, it->second, W).S) return true;
+    std::lock_guard<std::mutex> g(op.mu);
+    auto it = op.scratch.find(static_cast<void*>(st));
+    if (it != op.scratch.end()) {
+        if (held_scratch(op, it->second, W).S) return true;
+        if (W >= it->second.refused) return false;
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return false;
     }
-    try {
-        get_scratch(op, st, W);
-        return true;
-    } catch (const Error&) {
+    Scratch& sc = stream_scratch(op, st);
+    hipError_t e = hipErrorOutOfMemory;
+    ScratchW s;
+    if (scratch_sizes(op, W).total() <= wide_scratch_limit()) e = alloc_scratch(op, W, st, s);
+    if (e != hipSuccess) {
         (void)hipGetLastError();
+        if (e == hipErrorOutOfMemory) sc.refused = W;
         return false;
     }
+    keep_scratch(op, sc, W, s);
+    return true;
 }
 
 template <typename TS, typename TIO>

@@ -17,6 +17,7 @@ struct Scratch {
     ScratchW w[5];  // W = 1, 4, 16, 32, 48
     uint64_t last_use = 0;  // DeviceOp::use_clock at the stream's last product
     size_t bytes = 0;       // bytes held by the arrays of every width
+    int refused = 1 << 30;  // narrowest wide pass that was refused its scratch
 };
 
 constexpr int kMaxWidth = 48;  // widest pass
@@ -116,27 +117,37 @@ inline void clear_new_staging(void* S, const StagingLayout& lay, hipStream_t st)
     HIPCHECK(hipStreamDestroy(own));
 }
 
-// Allocate the scratch of one pass width, with its zero rows cleared before anything
-// else on `st`; returns its bytes.  `s` is set only when both have succeeded.
-inline size_t alloc_scratch(const DeviceOp& op, int W, hipStream_t st, ScratchW& s) {
+// Byte sizes of the three arrays of one pass width, each a multiple of 256.
+struct ScratchSizes {
+    size_t s, p, lp;
+    size_t total() const { return s + p + lp; }
+};
+inline ScratchSizes scratch_sizes(const DeviceOp& op, int W) {
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t pe = p_elem(op.storage);
-    const StagingLayout lay = staging(op, W);
-    const size_t sb = up(static_cast<size_t>(lay.zero_end));
-    const size_t pb = up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe);
-    const size_t lb = up(static_cast<size_t>(std::max<int64_t>(op.nlrows, 1)) * W * pe);
+    return {up(static_cast<size_t>(staging(op, W).zero_end)),
+            up(static_cast<size_t>(std::max<int64_t>(op.npartial, 1)) * W * pe),
+            up(static_cast<size_t>(std::max<int64_t>(op.nlrows, 1)) * W * pe)};
+}
+
+// Allocate the scratch of one pass width, with its zero rows cleared before anything
+// else on `st`.  Returns the status of the allocation; every other failure throws, and `s`
+// is set only when all has succeeded.
+inline hipError_t alloc_scratch(const DeviceOp& op, int W, hipStream_t st, ScratchW& s) {
+    const ScratchSizes z = scratch_sizes(op, W);
     ScratchW n;
-    HIPCHECK(hipMalloc(&n.S, sb + pb + lb));
+    const hipError_t e = hipMalloc(&n.S, z.total());
+    if (e != hipSuccess) return e;
     try {
-        clear_new_staging(n.S, lay, st);
+        clear_new_staging(n.S, staging(op, W), st);
     } catch (...) {
         (void)hipFree(n.S);
         throw;
     }
-    n.P = static_cast<char*>(n.S) + sb;
-    n.LP = static_cast<char*>(n.P) + pb;
+    n.P = static_cast<char*>(n.S) + z.s;
+    n.LP = static_cast<char*>(n.P) + z.p;
     s = n;
-    return sb + pb + lb;
+    return hipSuccess;
 }
 
 // Work lists of one launch (one H-matrix, or a batch of them).
