@@ -233,6 +233,17 @@ NoAllocPlan noalloc_plan(const DeviceOp& op, int W) {
     return pl;
 }
 
+// Usable bytes of that static scratch: HMX_NOALLOC_LIMIT lowers them, e.g. to exercise
+// the size checks on small operators; it never raises them.
+size_t noalloc_limit() {
+    size_t limit = kNoAllocScratchBytes;
+    if (const char* env = std::getenv("HMX_NOALLOC_LIMIT")) {
+        const long long v = std::atoll(env);
+        if (v >= 0 && static_cast<size_t>(v) < limit) limit = static_cast<size_t>(v);
+    }
+    return limit;
+}
+
 }  // namespace
 
 void device_destroy(DeviceOp* op) {
@@ -681,12 +692,13 @@ void device_build(HMatrix& h, int storage) {
         const int64_t fine_rows = op->nlrows;
         const int64_t rows = split_leaf_items(
             coarse, TK, pieces > 0 ? std::max(leaf_bytes / pieces, kMiB) : 0, csrc);
+        const size_t limit = noalloc_limit();
         bool refused = false;
         for (int W : {1, 4, 16}) {
             op->nlrows = fine_rows;
-            const bool fine_fits = noalloc_plan(*op, W).total <= kNoAllocScratchBytes;
+            const bool fine_fits = noalloc_plan(*op, W).total <= limit;
             op->nlrows = rows;
-            refused = refused || (!fine_fits && noalloc_plan(*op, W).total <= kNoAllocScratchBytes);
+            refused = refused || (!fine_fits && noalloc_plan(*op, W).total <= limit);
         }
         if (refused) {
             itemsB.swap(coarse);
@@ -1065,13 +1077,7 @@ void device_matvec_noalloc(HMatrix& h, int storage, const void* X, int64_t ldx, 
     if (nrhs <= 0) return;
     if (!X || !Y) throw Error(HMX_ERR_ARG, "null X or Y");
     if (ldx < h.n || ldy < h.m) throw Error(HMX_ERR_ARG, "leading dimension smaller than the size");
-    // HMX_NOALLOC_LIMIT lowers the usable part of the array (bytes), e.g. to
-    // exercise the size check on small operators; it never raises it
-    size_t limit = kNoAllocScratchBytes;
-    if (const char* env = std::getenv("HMX_NOALLOC_LIMIT")) {
-        const long long v = std::atoll(env);
-        if (v >= 0 && static_cast<size_t>(v) < limit) limit = static_cast<size_t>(v);
-    }
+    const size_t limit = noalloc_limit();
     DeviceOp& op = *h.dev[storage];
     DeviceGuard guard(op.device);
     hipStream_t st = static_cast<hipStream_t>(stream);
