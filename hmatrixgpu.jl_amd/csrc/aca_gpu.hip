@@ -238,13 +238,13 @@ __global__ __launch_bounds__(256) void k_copy_segs(const Seg* __restrict__ segs,
 // operation order is the host's (svd_recompress): reflector sums in the 64-lane
 // order of dot_lanes64, every other sum sequential in one lane, contraction
 // off, so the factors are bit-identical to the host recompression.  The
-// helpers are inlined: as called functions they made the kernels reserve 212 and
-// 184 VGPRs (2 waves per SIMD); inlined, 111 and 76, and the recompression is
-// 5% faster.
+// helpers are inlined: as called functions they made the kernels reserve up to 212
+// VGPRs, and the recompression was 5% slower (measured when two kernels of one wave
+// per block did all of it).
 struct RecTask {
     int64_t uoff, voff;  // ACA terms: U m x k, V' n x k, column-major, in the pool
     int64_t soff;        // scratch: M, Z, W, Z2 (k*k each), nrm, sig, ord, tu, tv (k each)
-    int64_t ooff;        // output: U' (m x r column-major) then V (r x n column-major)
+    int64_t ooff;        // output: U' (m x r column-major) then V (r x n row-major)
     int32_t m, n, k, r;
 };
 

@@ -864,9 +864,10 @@ void run(DeviceOp& op, const void* X, int64_t ldx, void* Y, int64_t ldy, int nrh
 // RHS width of a pass: one column -> VALU GEMV, up to 4 -> VALU 4-wide, more ->
 // MFMA passes of 16, 32 or 48 columns.  A pass reads the whole matrix, so the
 // fewest passes of at most 48 columns are taken, and of those the narrowest that
-// hold nrhs.  At N = 16,384 a pass of 16 / 32 / 48 takes 325 / 376 / 444 us (FP64),
-// 176 / 213 / 264 us (FP32) and 118 / 148 / 178 us (BF16): every wider pass beats the
-// narrow ones that it stands for, from 17 columns on (FP64 with 17: 376 against 560).
+// hold nrhs.  At N = 16,384 a pass of 16 / 32 / 48 takes 311 / 372 / 444 us (FP64),
+// 160 / 194 / 238 us (FP32) and 96 / 112 / 144 us (BF16): every wider pass beats the
+// narrow ones that it stands for, from 17 columns on (370, 193 and 108 us with 17,
+// against 621, 321 and 192 us for two passes of 16).
 int pass_width(int nrhs) {
     if (nrhs <= 4) return nrhs == 1 ? 1 : 4;
     const int passes = (nrhs + 47) / 48;

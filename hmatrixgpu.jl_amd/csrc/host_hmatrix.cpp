@@ -300,8 +300,9 @@ std::unique_ptr<HMatrix> build_hmatrix(const ClusterTree& T, const ClusterTree& 
     std::mutex slab_mu;
     std::vector<int64_t> rank(approx.size(), 0);
     if (opt->aca_device == 1) {
-        // batched ACA+ on the GPU with a rank capacity per block; recompression
-        // on host threads as blocks come back
+        // batched ACA+ on the GPU with a rank capacity per block; recompressed there
+        // too, or (for a tolerance below zero, which the device does not take) on host
+        // threads as blocks come back
         std::vector<AcaBlock> blocks(static_cast<size_t>(na));
         std::vector<int32_t> caps(static_cast<size_t>(na), std::max(1, opt->initial_rank));
         for (int64_t b = 0; b < na; b++) {

@@ -234,8 +234,14 @@ int hmx_hmatrix_release(hmx_hmatrix* h, int32_t storage_mask);
 /* Free the per-stream product scratch (see hmx_matvec) that `stream` holds, or
  * that every stream holds when all_streams != 0, for every materialised
  * precision, after synchronising those streams.  Each stream that has run a
- * product keeps about (n + R) * 16 * s_store + m * 16 * 4 bytes per RHS width
- * used (about 1.6 GB at N = 262,144 with FP32 storage and 16 RHS) until this
+ * product keeps, per pass width W used (1, 4, 16, 32 or 48 columns), the
+ * staging array of hmx_staging_layout, about (n + R) * W elements, and W partial
+ * sums (FP64, or FP32 for the other storages) per leaf-result row (one set of a
+ * leaf's rows for each piece that it is cut into) and far-field chunk row: 1.6 GB
+ * at N = 262,144 with FP32 storage and W = 16, 4.8 GB with W = 48.  The scratch of
+ * a wider pass serves the passes of 16 and 32 columns too, and one of 32 or 48 is
+ * allocated only within half of the free device memory (or HMX_WIDE_SCRATCH_LIMIT
+ * bytes); hmx_hmatrix_scratch_usage reports what is held.  It is kept until this
  * call, hmx_hmatrix_release or hmx_hmatrix_destroy; the next product on the
  * stream allocates it again.  At most HMX_SCRATCH_STREAMS streams (default 8)
  * hold scratch per materialised precision: a product on a further stream first
@@ -248,13 +254,13 @@ int hmx_hmatrix_release_scratch(hmx_hmatrix* h, void* stream, int32_t all_stream
  * it.  No reference counterpart (monitoring of the scratch above). */
 int hmx_hmatrix_scratch_usage(const hmx_hmatrix* h, int64_t* bytes, int64_t* entries);
 /* Size of the source/T staging array that one product pass of `width`
- * right-hand sides (1, 4 or 16; a product with nrhs > 16 runs ceil(nrhs / 48)
- * passes of 16, 32 or 48, the wider ones with two or three times the bytes of 16,
- * or passes of 16 where that memory is not to be had) allocates for an operator of `storage` precision with n source
- * rows and R stacked low-rank rows (sizes[4] of hmx_hmatrix_sizes): *rows rows
- * of *bytes / *rows bytes, of which [*zero_begin, *zero_end) must read zero
- * (cleared at allocation, and by hmx_matvec_noalloc on every call).  The
- * kernels read an array below 4 GiB through 32-bit buffer offsets and a larger
+ * right-hand sides (1, 4 or 16) allocates for an operator of `storage` precision
+ * with n source rows and R stacked low-rank rows (sizes[4] of hmx_hmatrix_sizes).
+ * A product with nrhs > 16 runs ceil(nrhs / 48) passes of 16, 32 or 48, the wider
+ * ones with two or three times the bytes of 16, or narrower passes where that
+ * memory is not to be had.  The array has *rows rows of *bytes / *rows bytes, of
+ * which [*zero_begin, *zero_end) must read zero (cleared at allocation, and by
+ * hmx_matvec_noalloc on every call).  The kernels read an array below 4 GiB through 32-bit buffer offsets and a larger
  * one through 64-bit global loads; rows are 32-bit indices, so
  * HMX_ERR_UNSUPPORTED from 2^31 rows.  No reference counterpart (memory
  * planning for the reference's Vx_buffer, hmatrix.jl:135). */
@@ -316,7 +322,9 @@ int hmx_hmatrix_destroy(hmx_hmatrix* h);
  * (H-matrix, stream), so concurrent calls on different streams are safe;
  * concurrent calls on one stream are ordered by the stream.  The first call on
  * a new stream allocates its scratch (hipMalloc), and so does the first with a
- * wider pass (nrhs 1, 2-4, 5-16, 17-32 and 33 or more differ). */
+ * wider pass (nrhs 1, 2-4, 5-16, 17-32 and 33 or more differ).  Under stream
+ * capture a product with nrhs > 4 allocates nothing once the stream has run any
+ * product with nrhs > 4. */
 int hmx_matvec(hmx_hmatrix* h, int32_t storage, const void* X, int64_t ldx, void* Y, int64_t ldy,
                int32_t nrhs, int32_t io_dtype, void* stream);
 
